@@ -243,7 +243,7 @@ int lowbit_w4_qkv_rope_rows(const void* x, const void* w, const void* s, int64_t
 /* Causal GQA attention: out[M][Hq * 128] for queries q [M][Hq][128] at positions[m] over cache rows 0..positions[m]
  * (at most L); scores scaled by `scale`, softmax and P.V in fp32. Cache rows past the largest position of the call
  * are never read into a result (they may hold anything, NaN included); rows up to it must be finite, since a
- * multi-token step reads whole 32-key blocks up to the largest position of the rows it groups. max_keys: an upper bound on positions[m] + 1 over
+ * multi-token step reads whole blocks of keys up to the largest position of the rows it groups. max_keys: an upper bound on positions[m] + 1 over
  * the calls that will run (sizes the launch; a captured graph keeps it; keys past it are still attended, by the last
  * key partition). Hq / Hkv in {1, 2, 4, 6, 7, 8}. workspace (optional, 16-byte aligned, at least 4096 bytes, no
  * initial contents needed; its first 4096 bytes are not used -- version 0.2 kept arrival counters there and needed

@@ -4,6 +4,8 @@
 // Qwen2RMSNorm, apply_rotary_pos_emb + StaticCache.update, scaled_dot_product_attention with a causal mask), with
 // the same fp16 roundings where the torch ops round.
 #include <algorithm>
+#include <cfloat>
+#include <climits>
 
 #include "kernels.hpp"
 
@@ -417,6 +419,257 @@ __global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, 
   for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(mine + 4 + 16 * dt + 4 * c) = o[dt];
 }
 
+// Causal GQA attention for prompts and long steps (the contract of attention_mfma): a workgroup of four waves takes
+// 32 RG query rows of one KV head (row = token * G + head-in-group) and walks the keys in blocks of 32 KG that its waves
+// share through LDS; a wave owns 32 rows (row group wave % RG) and 32 keys of every block (key group wave / RG), and the
+// key groups' sums are merged at the end. Per block and wave (v_mfma_f32_32x32x16_f16, lane l: j = l % 32, h = l / 32):
+//   S^T = K Q^T: A = 32 keys x 16 dims from LDS, B = the wave's 32 rows (registers). Lane (j, h) holds row j's scores of
+//   keys 8 (v / 4) + 4 h + v % 4, v = 0..15: two lanes a row.
+//   Online softmax in base 2 against a reference that follows the running maximum only when a score exceeds it by more
+//   than kAttnLag (the weights then reach 2^kAttnLag at most), so that the 64 accumulator registers are rescaled in the
+//   first blocks only and no lane exchange is needed in the others. The weights are split into an fp16 head and an fp16
+//   remainder (to ~2^-22) as in attention_mfma.
+//   O^T += V^T P^T: B = the weights as the lane holds them, i.e. contraction index 8 h + i of step s is key
+//   16 s + 8 (i / 4) + 4 h + i % 4; A = V^T from LDS by transposing reads (ds_read_b64_tr_b16).
+// K and V go from memory straight to LDS, one block ahead (K two: a block's scores are multiplied while the vector unit
+// evaluates the weights of the block before), with one barrier per block.
+// attention_mfma has a wave of 16 rows load its own K and V and wait for them in every block: L2 latency and reads bound
+// it. Here 32 RG rows share them; what is left is the matrix cores (three products per score and dim, the weights being
+// split), about level with the softmax's vector instructions, at two waves per SIMD (188 registers, 64 KB of LDS a
+// workgroup at KG = 2). Against 64 rows (RG = KG = 2), 128 rows (RG = 4, KG = 1) lengthen the serial walk of the last
+// rows: 3000 tokens 97 us against 81 (before K's second block ahead and the transposing reads), 700 tokens 27 against
+// 21; 32 rows (KG = 4) double the L2 reads (126 us) and win only where 64 rows leave CUs idle.
+// MI355X, 16 query / 2 KV heads, us (attention_mfma -> this): 3000 tokens 285 -> 76, 700 tokens 32.5 -> 17.2, 300 tokens
+// 16.4 -> 11.4, 128 tokens 11.1 -> 8.9; 512 tokens on 4096 cached 204 -> 53, 128 on 8000 125 -> 39 (KG = 4; 70 and 49
+// with KG = 2); 28 / 4 heads, 2048 tokens 230 -> 63.
+constexpr float kAttnLag = 8.f;
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
+template <int RG, int KG>
+__global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                                           const f16* __restrict__ v_cache,
+                                                           const int64_t* __restrict__ pos, f16* __restrict__ out, int M,
+                                                           int Hq, int Hkv, int L, float scale, int tiles,
+                                                           float* __restrict__ part) {
+  static_assert(RG * KG == 4, "four waves");
+  constexpr int kRows = 32 * RG, kKeys = 32 * KG;         // query rows of the workgroup, keys of a block
+  constexpr int kBuf = kKeys * kHeadDim * 2;                  // bytes of a block's K, and of its V
+  constexpr int NP = kKeys / 16;                              // 16-byte pieces a thread loads of K, and of V
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][K block, V block]
+  int* s_max = reinterpret_cast<int*>(smem);                  // the waves' last keys, before the first block is staged
+  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, tiles, part);
+  const int G = Hq / Hkv, P = gridDim.y, pid = blockIdx.y;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int j = lane & 31, h = lane >> 5;
+  // longest tiles first; every second round of workgroups in reverse, so that a CU's two workgroups add up alike
+  const int hk = blockIdx.x % Hkv, idx = blockIdx.x / Hkv, per = max(1, 256 / Hkv), rnd = idx / per;
+  const int at = rnd & 1 ? rnd * per + min(per, tiles - rnd * per) - 1 - (idx - rnd * per) : idx;
+  const int tile = tiles - 1 - at;
+  const int rgrp = wave % RG, kgrp = wave / RG;               // the wave's rows, and its keys of a block
+  const int row = kRows * tile + 32 * rgrp + j, m = row / G, g = row - m * G;
+  const bool live = m < M;
+  const int pr = live ? (int)min((int64_t)L - 1, pos[m]) : -1;    // last key the row attends
+  int wmax = pr, wmin = live ? pr : INT_MAX;                  // the wave's last key, and its rows' first last key
+#pragma unroll
+  for (int o = 1; o < 32; o <<= 1) {
+    wmax = max(wmax, __shfl_xor(wmax, o, 64));
+    wmin = min(wmin, __shfl_xor(wmin, o, 64));
+  }
+  wmax = __builtin_amdgcn_readfirstlane(wmax);
+  wmin = __builtin_amdgcn_readfirstlane(wmin);
+  if (lane == 0) s_max[wave] = wmax;
+  __syncthreads();
+  const int gmax = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+  __syncthreads();
+  const int ch = ((gmax + 1 + P - 1) / P + kKeys - 1) / kKeys * kKeys;
+  const int kbeg = pid * ch, kend = min(gmax + 1, kbeg + ch);
+  // q of row j, dims 16 ks + 8 h .. + 7; a negative scale is moved into q (exact), so that score order is weight order
+  const uint32_t flip = scale < 0.f ? 0x80008000u : 0u;
+  // base-2 score scale; held above 0, so that a masked score of -inf stays -inf (scale 0: every weight is 2^~0 = 1)
+  const float c2 = fabsf(scale) * 1.44269504088896340736f < FLT_MIN ? FLT_MIN : fabsf(scale) * 1.44269504088896340736f;
+  f16x8 qf[8];
+  const f16* qrow = q + ((size_t)min(m, M - 1) * Hq + hk * G + g) * kHeadDim + 8 * h;
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    u32x4 t = load16(qrow + 16 * ks);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) t[e] ^= flip;
+    qf[ks] = __builtin_bit_cast(f16x8, t);
+  }
+  const uint8_t* kh = reinterpret_cast<const uint8_t*>(k_cache + (size_t)hk * L * kHeadDim);
+  const uint8_t* vh = reinterpret_cast<const uint8_t*>(v_cache + (size_t)hk * L * kHeadDim);
+  // K and V rows go straight to LDS as they are, 256 bytes each: this thread's pieces are 16 bytes of keys tid / 16 + 16 u,
+  // slot tid % 16 of the row, whose 16-byte pieces are permuted by the key: K's so that the 32 rows of a fragment read
+  // meet different banks, V's so that the four rows of a transposing read do. Rows past the last attended key (never
+  // written, maybe NaN) are clamped to it: their weight 0 must meet finite values
+  const int kk = tid >> 4, kp = tid & 15;
+  const uint32_t dst = lds_addr(smem) + 1024 * wave;
+  auto load = [&](const uint8_t* rows, int kb, int piece, uint32_t at) {   // (a block past the last one: the last key)
+    const int k0 = min(kb, gmax), lim = gmax - k0;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(rows + (size_t)k0 * 256, kBuf);
+#pragma unroll
+    for (int u = 0; u < NP; ++u) dma16(rs, min(kk + 16 * u, lim) * 256 + 16 * piece, dst + at + 4096 * u);
+  };
+  auto vswz = [](int key) { return 4 * (key & 3) + 2 * ((key >> 2) & 1); };
+  auto load_k = [&](int kb, uint32_t base) { load(kh, kb, kp ^ kk, base); };
+  auto load_v = [&](int kb, uint32_t base) { load(vh, kb, kp ^ vswz(kk), base + kBuf); };
+  // LDS offsets in a buffer. Both permutations are an exclusive-or of address bits 4..7 applied to the running offset, so
+  // one register holds each family. K: row 32 kgrp + j, pieces 2 s + h. V: transposing 8-byte reads (16 lanes i get column
+  // i of the 4 keys x 16 dims whose 8-byte pieces they address): key 4 h + i / 4, dims 16 (l / 16 % 2) + 4 (i % 4)
+  const uint32_t kr = (32 * kgrp + j) * 256 + 16 * (h ^ (j & 15));
+  const int vk = 4 * h + ((lane & 15) >> 2), vp = 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1);
+  const uint32_t vr = kBuf + (32 * kgrp + vk) * 256 + 16 * (vp ^ vswz(vk)) + 8 * (lane & 1);
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  auto v_frag = [&](uint32_t at) {                            // keys at .. and at + 8 rows, this lane's dim
+    typedef __attribute__((address_space(3))) s16x4* lds_ptr;
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + at));
+    const s16x4 c = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + at + 2048));
+    return __builtin_bit_cast(f16x8, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  float ref = -INFINITY, lsum = 0.f;                          // reference (base 2), the lane's share of the weights' sum
+  f32x16 o[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) o[dt][v] = 0.f;
+
+  const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  f32x16 st = zero;                                           // scores of the wave's 32 keys of a block
+  auto scores = [&](uint32_t base, int s0, int s1) {          // dims 16 s0 .. 16 s1 of them
+#pragma unroll
+    for (int s = s0; s < s1; ++s)
+      st = __builtin_amdgcn_mfma_f32_32x32x16_f16(*reinterpret_cast<const f16x8*>(smem + ((kr + base) ^ (32 * s))), qf[s], st,
+                                                  0, 0, 0);
+  };
+  // one block: the weights of its scores, the weights times V and the next block's scores (its K lies in the other
+  // buffer), whose products run while the vector unit evaluates the weights
+  auto block = [&](uint32_t base, int kb) {                   // kb: the wave's first key
+    if (kb + 31 > min(wmin, kend - 1)) {                      // some row attends part of these keys only (uniform)
+      const int last = min(pr, kend - 1) - kb - 4 * h;        // a key at or below it counts
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        if (8 * (v >> 2) + (v & 3) > last) st[v] = -INFINITY;
+    }
+    float bm = st[0];
+#pragma unroll
+    for (int v = 1; v < 16; ++v) bm = fmaxf(bm, st[v]);
+    if (__any(bm * c2 > ref + kAttnLag)) {                    // (uniform; either lane of a row)
+      const float nm = fmaxf(ref, fmaxf(bm, __shfl_xor(bm, 32, 64)) * c2);   // -inf while the row has seen no key
+      const float corr = nm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(ref - nm);
+      ref = nm;
+      lsum *= corr;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) o[dt] *= corr;
+    }
+    const float sub = ref == -INFINITY ? 0.f : ref;
+    const f32x16 sc = st;
+    st = zero;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {                             // 16 keys: head and remainder of their weights, then V
+      u32x4 ph, pl;
+      float ps[2] = {0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const f32x2 p = {__builtin_amdgcn_exp2f(fmaf(sc[8 * s + 2 * i], c2, -sub)),
+                         __builtin_amdgcn_exp2f(fmaf(sc[8 * s + 2 * i + 1], c2, -sub))};
+        ps[0] += p[0];
+        ps[1] += p[1];
+        const f16x2 head = __builtin_convertvector(p, f16x2);
+        const f32x2 rest = {p[0] - (float)head[0], p[1] - (float)head[1]};
+        ph[i] = as_u32(head);
+        pl[i] = as_u32(__builtin_convertvector(rest, f16x2));
+      }
+      lsum += ps[0] + ps[1];
+      scores(base ^ (2 * kBuf), 4 * s, 4 * s + 4);            // (past the last block: of stale K, never used)
+      f16x8 va[4];
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt) va[dt] = v_frag(((vr + base) ^ (64 * dt)) + 4096 * s);
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(f16x8, ph), o[dt], 0, 0, 0);
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[dt], __builtin_bit_cast(f16x8, pl), o[dt], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+
+  // buffer b holds block i's V and block i + 1's K is in the other one, whose V slot takes block i + 1 at the end; the K
+  // of block i + 2 replaces that of block i, whose scores are in registers
+  if (kbeg < kend) {
+    load_k(kbeg, 0);
+    load_k(kbeg + kKeys, 2 * kBuf);
+    load_v(kbeg, 0);
+  }
+  lds_wait_barrier<0>();
+  if (kbeg < kend) scores(0, 0, 8);
+  lds_barrier();                                              // every wave has read the first K
+  uint32_t b = 0;
+  for (int kb = kbeg; kb < kend; kb += kKeys, b ^= 2 * kBuf) {
+    const bool more = kb + kKeys < kend;
+    if (more) {
+      load_k(kb + 2 * kKeys, b);
+      load_v(kb + kKeys, b ^ (2 * kBuf));
+    }
+    block(b, kb + 32 * kgrp);
+    lds_wait_barrier<0>();                                    // the K and V requested above are visible
+  }
+  lsum += __shfl_xor(lsum, 32, 64);
+  if constexpr (KG > 1) {                                     // the key groups' sums, through LDS, into key group 0
+    constexpr int kRec = 66 * 64 * 4;                         // a wave's sums, reference and weight sum
+    float* mine = reinterpret_cast<float*>(smem + (size_t)((kgrp - 1) * RG + rgrp) * kRec) + lane;
+    if (kgrp > 0) {
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) mine[64 * (16 * dt + v)] = o[dt][v];
+      mine[64 * 64] = ref;
+      mine[65 * 64] = lsum;
+    }
+    lds_barrier();
+    if (kgrp > 0) return;
+    for (int g2 = 1; g2 < KG; ++g2) {
+      const float* theirs = reinterpret_cast<const float*>(smem + (size_t)((g2 - 1) * RG + rgrp) * kRec) + lane;
+      const float r2 = theirs[64 * 64], nm = fmaxf(ref, r2);
+      const float c0 = ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ref - nm);
+      const float c1 = r2 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(r2 - nm);
+      ref = nm;
+      lsum = lsum * c0 + theirs[65 * 64] * c1;
+#pragma unroll
+      for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[dt][v] = o[dt][v] * c0 + theirs[64 * (16 * dt + v)] * c1;
+    }
+  }
+  if (!live) return;
+  // lane (j, h) holds O^T[32 dt + 8 (v / 4) + 4 h + v % 4][row j]
+  if (P == 1) {
+    f16* dst = out + ((size_t)m * Hq + hk * G + g) * kHeadDim + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+      for (int v = 0; v < 16; v += 4) {
+        const f16x2 lo = {(f16)(o[dt][v] / lsum), (f16)(o[dt][v + 1] / lsum)};
+        const f16x2 hi = {(f16)(o[dt][v + 2] / lsum), (f16)(o[dt][v + 3] / lsum)};
+        *reinterpret_cast<uint2*>(dst + 32 * dt + 2 * v) = make_uint2(as_u32(lo), as_u32(hi));
+      }
+    return;
+  }
+  // the record's maximum and sum are natural-base ones: ref / log2(e)
+  float* mine = part + (((size_t)(m * Hkv + hk) * P + pid) * G + g) * kAttnRec;
+  if (h == 0) {
+    mine[0] = ref * 0.69314718055994530942f;
+    mine[1] = lsum;
+  }
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+    for (int v = 0; v < 16; v += 4)
+      *reinterpret_cast<f32x4*>(mine + 4 + 32 * dt + 2 * v + 4 * h) = f32x4{o[dt][v], o[dt][v + 1], o[dt][v + 2], o[dt][v + 3]};
+}
+
 // fp16 GEMV for the (tied) lm_head, M <= 4: y[m][n] = fp16(sum_k x[m][k] W[n][k]), W fp16 [N][K] row-major, fp32
 // accumulation. A bandwidth kernel: the workgroup stages x[M][K] in LDS once (one barrier), then each wave streams
 // RW weight rows with 16-byte non-temporal loads (lane l takes k = 512 c + 8 l .. + 7 of chunk c, so every load is
@@ -787,11 +1040,48 @@ hipError_t launch_attention_mfma(const f16* q, const f16* k, const f16* v, const
   return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
                 Hq);
 }
+// prompts: one workgroup per (KV head, 32 RG query rows, key partition); partitions while the workgroups number fewer
+// than kAttnPromptTargetGroups, at most one per kAttnPromptMinKeys of max_keys, within the workspace
+template <int RG, int KG>
+hipError_t launch_attention_prompt(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M,
+                                   int Hq, int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes,
+                                   hipStream_t st) {
+  const int G = Hq / Hkv;
+  const int tiles = (int)(((long)M * G + 32 * RG - 1) / (32 * RG));
+  const long wgs = (long)tiles * Hkv;
+  int P = 1;
+  if (ws && ws_bytes > kAttnCounterBytes && wgs < kAttnPromptTargetGroups && max_keys >= 2 * kAttnPromptMinKeys) {
+    P = (int)std::min<long>({(kAttnPromptTargetGroups + wgs - 1) / wgs,
+                             (max_keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys, (long)kAttnMaxParts});
+    const size_t per = (size_t)M * Hq * kAttnRec * sizeof(float);
+    P = (int)std::max<size_t>(1, std::min<size_t>((size_t)P, (ws_bytes - kAttnCounterBytes) / per));
+  }
+  float* part = ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kAttnCounterBytes) : nullptr;
+  const size_t lds = std::max<size_t>((size_t)2 * 2 * 32 * KG * kHeadDim * 2, (size_t)(KG - 1) * RG * 66 * 256);
+  if (lds > 65536) {
+    static const hipError_t attr = allow_lds(attention_prompt<RG, KG>, lds);
+    if (attr != hipSuccess) return attr;
+  }
+  hipError_t e = launch(attention_prompt<RG, KG>, dim3((unsigned)wgs, P), dim3(256), lds, st, q, k, v, pos, out, M, Hq,
+                        Hkv, L, scale, tiles, part);
+  if (e != hipSuccess || P == 1) return e;
+  const long threads = (long)M * Hq * kHeadDim;
+  return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
+                Hq);
+}
 }  // namespace
 
 hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
                             int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
-  if ((long)M * (Hq / Hkv) >= kAttnMfmaMinRows)
+  const long rows = (long)M * (Hq / Hkv);
+  // the prompt kernel's longer prologue and merge pay from about 384 rows (16 / 2 heads, 48 tokens on 600 cached: level
+  // at 12.9 us; 28 / 4 heads, 64 on 1000: 21.7 -> 17.1; below: 16 tokens on 512 cached 9.0 against 11.4 us)
+  if (rows >= kAttnPromptMinRows) {
+    if ((rows + 63) / 64 * Hkv < kAttnPromptWide && max_keys >= kAttnPromptLongKeys)
+      return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+  }
+  if (rows >= kAttnMfmaMinRows)
     return launch_attention_mfma(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
   if ((long)M * Hkv < 64)                                     // few tokens: one query head per block, short steps
     return launch_attention<1, 32>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);

@@ -287,6 +287,13 @@ constexpr size_t kAttnCounterBytes = 4096;
 // splits keys while its waves number fewer than kAttnMfmaTargetWaves
 constexpr int kAttnMfmaMinRows = 32;
 constexpr int kAttnMfmaTargetWaves = 512;
+// the prompt attention takes steps with at least kAttnPromptMinRows query rows per KV head, with 64 rows a workgroup, or
+// 32 where those leave CUs idle (fewer than kAttnPromptWide workgroups) and there are keys to share out
+constexpr int kAttnPromptMinRows = 384;
+constexpr int kAttnPromptWide = 160;
+constexpr int kAttnPromptLongKeys = 1024;
+constexpr int kAttnPromptTargetGroups = 512;
+constexpr int kAttnPromptMinKeys = 128;
 constexpr int kAttnManyBlocks = 512;      // from this many blocks on, at most 4 waves per block
 constexpr int kMaxSplits = 32;
 constexpr size_t kCounterBytes = 16384;
