@@ -55,10 +55,9 @@ const char* lowbit_version(void);
 
 /* Process-wide launch-shape override of the MFMA-layout kernels, for tuning sweeps. waves_per_group: the M <= 8
  * GEMV's waves per workgroup (0 = automatic, else 1, 2, 4, 8 or 16; clamped to what the register budget allows); for
- * the prefill GEMM the tile shape (1: 64 activation rows / 4 waves, 2: 64 / 8 waves, 4: 128 / 4 waves, 8: 128 / 8
- * waves, which is never built and falls back to 4 waves). ring: chunk slots in flight per wave (0 = automatic, else
- * 2, 3, 4 or 8: the GEMV uses 4 or 8, 8 only for M <= 2; the MFMA GEMM 2, 3 or 4; the prefill GEMM 2 or 3, and 4 =
- * 2 with a two-chunk activation lookahead). k_splits: workgroups the MFMA and prefill GEMMs split K over
+ * the prefill GEMM the tile shape (1 or 2: 64 activation rows, 4 or 8: 128; 128 weight rows and 4 waves). ring: chunk
+ * slots in flight per wave (0 = automatic, else 2, 3, 4 or 8: the GEMV uses 4 or 8, 8 only for M <= 2; the MFMA GEMM
+ * 2, 3 or 4; the prefill GEMM has one depth and ignores it). k_splits: workgroups the MFMA and prefill GEMMs split K over
  * (0 = automatic, 1..32; bounded by the workspace and by K / 128); for the M <= 8 GEMV, workgroups sharing one
  * 16-row tile (1, 2 or 4, owning 16, 8 or 4 rows each; honoured with one tile per wave, K / 128 a multiple of it and
  * no silu-mul or RoPE epilogue, which pair rows r and r + 8; other values leave the GEMV's choice automatic).
@@ -177,8 +176,9 @@ int lowbit_w4_linear_fused(const void* x, const void* w, const void* s, void* y,
  * multiples of 128), reading the int4 weights directly, with the same epilogues as lowbit_w4_linear_fused. Replaces
  * the reference's prefill path, dequantize to fp16 + cuBLAS (lowbit/ops.py:126-135,163-178): the weights multiplied
  * are exactly the dequantized fp16 values. The workspace (optional, as for lowbit_w4_gemm_mfma: counters zeroed before
- * the first call and left zero) lets K split across workgroups when the tiles alone do not fill the GPU; partial sums
- * take S * M * N * 4 bytes after the counters, and the split count is lowered to what fits. Requires
+ * the first call and left zero) lets K split across workgroups when the tiles alone do not fill the GPU; the partial
+ * sums of the split tiles (at most 96 KB a tile and split) follow the counters, and the split count is lowered to what
+ * fits. Requires
  * (M + 128) * K * 2 < 2^31. */
 int lowbit_w4_gemm_prefill(const void* x, const void* w, const void* s, void* y, int64_t M, int64_t N, int64_t K,
                            int64_t group, int epilogue, const void* aux, void* workspace, size_t workspace_bytes,

@@ -225,6 +225,12 @@ __device__ __forceinline__ void dma16_nt(__amdgpu_buffer_rsrc_t r, int voffset, 
                "s"(lds)
                : "memory", "m0");
 }
+// dma16 with a wave-uniform part of the offset in a scalar register (voffset + soffset within the resource)
+__device__ __forceinline__ void dma16_s(__amdgpu_buffer_rsrc_t r, int voffset, int soffset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds" ::"v"(voffset), "s"(r),
+               "s"(soffset), "s"(lds)
+               : "memory", "m0");
+}
 #pragma clang diagnostic pop
 // Wait until at most N of this wave's vector-memory operations are outstanding, then read 16 bytes at LDS byte
 // `addr`. The read and its own wait sit in the same statement, so the value is complete when the statement ends and

@@ -9,23 +9,33 @@
 //   B (32 k x 16 activation rows): x[m0 + 16 mt + r][128 c + 32 q + 8 s + 0..7], 16 bytes from LDS.
 //   D: lane l holds y[m0 + 16 mt + r][16 t + 4 q + v], v = 0..3.
 //
-// Workgroup: 4 waves, each owning PT 16-row tiles (64 PT weight rows per workgroup; PT = 4, or 2 or 1 when the grid
-// would leave CUs idle), against 16 MT activation rows.
-// Every wave decodes only its own rows, so no weight is decoded twice; the activation chunk is loaded once per
-// workgroup (16 bytes per thread and row piece) and shared through LDS, double buffered with one barrier per 128-k
-// chunk. LDS rows are 256 bytes with the 16-byte column blocks XOR-swizzled by the row (block b of row m at
-// b ^ (m % 16)), so both the stores of a row and the 16-row fragment reads hit 16 different bank groups.
-// Weight pieces and scales run D chunks ahead in registers; the next chunk of x is requested before the current
-// chunk's MFMAs and written to LDS after them. Buffer loads make tails free: rows past N, chunks past the split's
-// range and activation rows past M read zeros.
+// Workgroup: 4 waves, each owning PT 16-row tiles (64 PT weight rows per workgroup) against 16 MT activation rows. Every
+// wave decodes only its own rows, so no weight is decoded twice in a workgroup; a 128-k chunk of x goes straight from
+// memory to LDS (direct-to-LDS loads, no registers) and is shared by the waves, double buffered. LDS rows are 256 bytes,
+// their 16-byte blocks permuted by the row (xswz: block b of row m at b ^ xswz(m % 16)), so that a fragment's 16 rows
+// meet different banks. Rows past N and activation rows past M read zeros or are never stored.
 //
-// Work items (tile = 256 rows x 16 MT activation rows, times S splits of K) are numbered with the split fastest, then
-// the activation group, then the row group, and the workgroup -> item map puts consecutive items on the same XCD
-// (workgroup i runs on XCD i % 8), so the workgroups that share weight rows share that XCD's L2. With S > 1 each
-// workgroup writes fp32 partials to the workspace (agent-coherent stores); the last to arrive on a per-tile counter
-// adds them in split order, applies the epilogue and resets the counter, as in the skinny kernel.
+// Pipeline: the chunk is walked in groups of two activation tiles; while a group's 2 PT MFMAs run, the next group's B
+// fragments are read and a share of the next k-step's A fragments decoded, across the chunk's end too, and one barrier per
+// chunk, which waits for x alone, leaves the weights of the chunk after next in flight. The version before (chunk decoded
+// whole, fragment reads waited for as they were issued, x through registers, a barrier that drained every load) left the
+// matrix cores 31% busy at 2048 x 3584 x 18944; this one keeps them 45-50% busy there, at the clock that the power limit
+// leaves (1.8-2.0 GHz; MFMAs with the decode's vector instructions between them and nothing else reach 1.6 PFLOP/s).
+// MI355X, graph-timed, cold weights, rows x K x N, us (before -> now, dequantize + hipBLASLt): 128 x 3584 x 18944 37.9 ->
+// 28.7 (63.5); 333 x 2048 x 11008 32.6 -> 30.3 (41.6); 333 x 11008 x 2048 46.8 -> 30.7 (52.4); 512 x 18944 x 3584 104 ->
+// 84 (203); 700 x 2048 x 22016 81 -> 73 (102); 1000 x 3584 x 18944 182 -> 149 (164); 2048 x 3584 x 18944 354 -> 282 (341).
+// Not kept: the same loop on 32x32x16 MFMAs (271-294 at 2048 x 3584 x 18944, more power per product), 8 tiles x 4
+// per wave (registers spill; the compiler moves accumulators between register files at 16), 8-wave workgroups.
+//
+// Work items: the tiles that fill whole rounds of the chip one workgroup each, the rest with K split S ways
+// (plan_gemm_prefill), activation groups fastest, then row groups, and the workgroup -> item map puts consecutive items
+// on the same XCD (workgroup i runs on XCD i % 8), so the workgroups that share weight rows share that XCD's L2. The
+// splits of a tile write fp32 partials to the workspace (agent-coherent stores); the last to arrive on the tile's counter
+// adds them in split order and resets the counter, as in the skinny kernel.
 #include <algorithm>
 #include <climits>
+#include <type_traits>
+#include <utility>
 
 #include "kernels.hpp"
 
@@ -33,86 +43,102 @@ namespace lowbit {
 
 namespace {
 
+// f(integral_constant 0) .. f(integral_constant N - 1)
+template <int... I, typename F>
+__device__ __forceinline__ void unrolled_seq(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void unrolled(F&& f) {
+  unrolled_seq(std::make_integer_sequence<int, N>{}, f);
+}
 
-__device__ __forceinline__ int swz(int row, int blk) { return row * 16 + (blk ^ (row & 15)); }   // 16-byte slot
+constexpr int xswz(int r) { return ((r & 3) << 2) | (r >> 2); }
 
 }  // namespace
 
-// Waves per SIMD the register allocation must leave room for: 2 for the 4-tile, 2-slot shapes (at most 256 registers
-// a wave, so two 4-wave workgroups share a CU), which fit in that budget without spilling; 1 for the 8-tile and 3-slot
-// shapes, which do not. Without the bound hipcc gave the 4 x 4-tile shape 260 registers (188 + 72 accumulation
-// registers): one workgroup per CU, and 3B gate|up at 2048 rows took 455 us instead of 249 (MI355X, cold weights).
-constexpr int prefill_min_waves(int MT, int D) { return MT == 4 && D == 2 ? 2 : 1; }
-
-template <int MT, int D, int NW, int XL, int PT, bool ROPE>
-__global__ __launch_bounds__(64 * NW, prefill_min_waves(MT, D)) void gemm_prefill(const f16* __restrict__ x, const uint8_t* __restrict__ w,
-                                                    const f16* __restrict__ s, f16* y, int M, int N, int K, int G,
-                                                    int S, int MG, int items, uint32_t* __restrict__ ctr,
-                                                    float* __restrict__ part, Epilogue epi) {
+template <int MT, int PT, bool ROPE>
+__global__ __launch_bounds__(256, 2) void gemm_prefill(
+    const f16* __restrict__ x, const uint8_t* __restrict__ w, const f16* __restrict__ s, f16* y, int M, int N, int K,
+    int G, int S, int MG, int full, int items, uint32_t* __restrict__ ctr, float* __restrict__ part, Epilogue epi) {
   constexpr int kXBuf = 16 * MT * 256;                      // one staged chunk of x
-  constexpr int kRows = 16 * PT * NW;                       // weight rows per workgroup
-  args_in_sgprs(x, w, s, y, M, N, K, G, S, MG, items, ctr, part, epi.aux);
-  constexpr int kThreads = 64 * NW;
+  constexpr int kRows = 64 * PT;                            // weight rows per workgroup
+  args_in_sgprs(x, w, s, y, M, N, K, G, S, MG, full, items, ctr, part, epi.aux);
+  constexpr int kThreads = 256;
   constexpr int XP = 16 * MT * 16 / kThreads;               // 16-byte x pieces per thread and chunk
   static_assert(XP >= 1 && XP * kThreads == 16 * MT * 16, "x pieces must divide evenly");
-  static_assert(D == 2 || XL == 1, "a 3-deep weight ring runs with a one-chunk x lookahead");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
 
-  // workgroup -> work item: consecutive items on one XCD
-  const int per = items >> 3, rem = items & 7, xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+  // workgroup -> work item: first `full` whole tiles, then the others S splits each; consecutive items on one XCD (full
+  // is a multiple of 8 unless it is all the tiles or none)
+  const bool whole = (int)blockIdx.x < full;
+  const int b0 = whole ? blockIdx.x : blockIdx.x - full, n_items = whole ? full : items - full;
+  const int per = n_items >> 3, rem = n_items & 7, xcd = b0 & 7, idx = b0 >> 3;
   const int item = xcd < rem ? xcd * (per + 1) + idx : rem * (per + 1) + (xcd - rem) * per + idx;
-  const int sp = item % S, tile = item / S, mg = tile % MG, ng = tile / MG;
+  if (whole) S = 1;
+  const int sp = item % S, tile = whole ? item : full + item / S, mg = tile % MG, ng = tile / MG;
   const int m0 = 16 * MT * mg, n0 = kRows * ng;
   const int ntiles = (N + 15) >> 4, KC = K >> 7, KG = K / G, cpg = G >> 7;
   const int cb = (int)((int64_t)KC * sp / S), ce = (int)((int64_t)KC * (sp + 1) / S);
   const int nsteps = ce - cb;
   const size_t tile_bytes = (size_t)8 * K;
 
-  __amdgpu_buffer_rsrc_t wr[PT];
-  int woff[PT], wstep[PT], soff[PT];
+  // Weight rows past N read other rows' nibbles or zeros; their scales lie past the end (zeros) and their outputs are not
+  // stored. The uniform part of an offset is in the resource's base, so one register serves all tiles. Chunks past the
+  // range are clamped to its last one and never consumed.
+  const uint8_t* wp[PT];
+  int wrows[PT], tc[PT];                                    // (uniform)
 #pragma unroll
   for (int i = 0; i < PT; ++i) {
     const int t = n0 / 16 + PT * wave + i;
-    const int tc = min(t, ntiles - 1);
-    const int rows = t < ntiles ? min(16, N - 16 * t) : 0;
-    wr[i] = make_rsrc(w + tc * tile_bytes, (uint32_t)(rows * (K / 2)));
-    woff[i] = r < rows ? 64 * r + 16 * q : kOutOfRange;
-    wstep[i] = r < rows ? rows * 64 : 0;
-    soff[i] = r < rows ? 2 * (16 * t + r) * KG : kOutOfRange;   // the scale of this lane's A row
+    tc[i] = min(t, ntiles - 1);
+    wrows[i] = t < ntiles ? min(16, N - 16 * t) : 0;
+    wp[i] = w + tc[i] * tile_bytes;
   }
-  const __amdgpu_buffer_rsrc_t sr = make_rsrc(s, (uint32_t)N * (uint32_t)KG * 2u);
-  const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)M * (uint32_t)K * 2u);
-  int xoff[XP], xslot[XP];                                  // piece tid + kThreads u: row p / 16, block p % 16
-#pragma unroll
-  for (int u = 0; u < XP; ++u) {
-    const int pc = tid + kThreads * u;
-    xoff[u] = ((m0 + (pc >> 4)) * K + 8 * (pc & 15)) * 2;
-    xslot[u] = 16 * swz(pc >> 4, pc & 15);
-  }
+  const int woff = 64 * r + 16 * q, soff = 2 * r * KG;
+  // piece tid + kThreads u of a staged chunk is slot p % 16 of row p / 16, which holds the row's 16-byte block
+  // slot ^ xswz(row % 16) (kThreads is a multiple of 256, so that block is the same for every u); each u has a resource
+  // of its own, from its first row's chunk to the end of x (rows past M read zeros)
+  const int xoff = ((tid >> 4) * K + 8 * ((tid & 15) ^ xswz((tid >> 4) & 15))) * 2;
+  const uint32_t xdst = lds_addr(smem) + 1024 * wave;
 
-  u32x4 rw[D][PT], rx[XL][XP];
-  uint32_t rs[D][PT];
+  u32x4 rw[2][PT];
+  uint32_t rs[2][PT];
   const uint32_t gmagic = cpg == 1 ? 0u : (uint32_t)(0xFFFFFFFFu / (uint32_t)cpg) + 1u;   // c / cpg == mulhi(c, gmagic)
-  auto issue_w = [&](int d, int c) {
-    const bool live = c < ce;
+  auto issue_w = [&](int d, int chunk) {                    // 2 PT loads (lds_wait_barrier counts them)
+    const int c = min(chunk, ce - 1);
     const int g = cpg == 1 ? c : (int)__umulhi((uint32_t)c, gmagic);
 #pragma unroll
     for (int i = 0; i < PT; ++i) {
-      rw[d][i] = buffer_load16(wr[i], live ? woff[i] + c * wstep[i] : kOutOfRange);   // re-read by other m-groups
-      rs[d][i] = buffer_load2(sr, live ? soff[i] + 2 * g : kOutOfRange);
+      const int at = c * wrows[i] * 64;                     // (weights are re-read by other m-groups: default policy)
+      rw[d][i] = buffer_load16(make_rsrc(wp[i] + at, (uint32_t)(wrows[i] * (K / 2) - at)), woff);
+      const int sat = 16 * tc[i] * KG + g;
+      rs[d][i] = buffer_load2(make_rsrc(s + sat, (uint32_t)(N * KG - sat) * 2u), soff);
     }
   };
-  auto issue_x = [&](int e, int c) {
+  // the activation rows of a full tile share one resource, the row part of the offset in a scalar register; the last,
+  // ragged tile takes one per u, cut off at the end of x (a scalar offset past the end would escape the bounds check)
+  const bool ragged = m0 + 16 * MT > M;
+  const uint8_t* xtile = reinterpret_cast<const uint8_t*>(x) + (size_t)m0 * K * 2;
+  const int ustep = kThreads / 8 * K;                       // bytes from one u's rows to the next one's
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(xtile, (uint32_t)(16 * MT * K * 2));
+  auto issue_x = [&](int b, int chunk) __attribute__((always_inline)) {   // chunk of x straight into LDS buffer b
+    const int c = min(chunk, ce - 1);
+    if (!ragged) {
+      int at = 256 * c;
 #pragma unroll
-    for (int u = 0; u < XP; ++u) rx[e][u] = buffer_load16(xr, c < ce ? xoff[u] + 256 * c : kOutOfRange);
-  };
-  auto stage_x = [&](int e, int b) {
+      for (int u = 0; u < XP; ++u, at += ustep) dma16_s(xr, xoff, at, xdst + b * kXBuf + 16 * kThreads * u);
+    } else {
 #pragma unroll
-    for (int u = 0; u < XP; ++u) *reinterpret_cast<u32x4*>(smem + b * kXBuf + xslot[u]) = rx[e][u];
+      for (int u = 0; u < XP; ++u) {
+        const int left = max(0, M - m0 - kThreads / 16 * u) * 2 * K - 256 * c;
+        dma16(make_rsrc(xtile + (size_t)u * ustep + 256 * c, (uint32_t)max(0, left)), xoff,
+              xdst + b * kXBuf + 16 * kThreads * u);
+      }
+    }
   };
 
   f32x4 acc[PT][MT];
@@ -124,252 +150,280 @@ __global__ __launch_bounds__(64 * NW, prefill_min_waves(MT, D)) void gemm_prefil
   const f16x2 m1032 = {(f16)-1032.0f, (f16)-1032.0f}, m72 = {(f16)-72.0f, (f16)-72.0f};
   const f16x2 inv16 = {(f16)0.0625f, (f16)0.0625f};
   const DecodeRegs dc = decode_regs();                      // masks and magic in registers: v_and_or_b32
-  // one chunk: the 16 A fragments (4 tiles x 4 k-steps) are decoded first; then per activation tile its 4 B
-  // fragments are read and 16 MFMAs issued, so at most two tiles' B fragments are live
-  auto consume = [&](int d, int b) {
-    f16x8 a[PT][4];
+  int xrd[4];                                               // lane (r, q): block 4 q + st of row r
 #pragma unroll
-    for (int i = 0; i < PT; ++i) {
-      const f16 sv = __builtin_bit_cast(f16, (uint16_t)rs[d][i]);
-      const f16x2 sc = {sv, sv};
-#pragma unroll
-      for (int st = 0; st < 4; ++st) {                      // (u - 8) exact, times the scale: one rounding
-        const uint32_t wd = rw[d][i][st], w8 = wd >> 8;
-        const f16x2 p0 = (as_f16x2((wd & dc.lo) | dc.magic) + m1032) * sc;
-        const f16x2 p1 = (as_f16x2((wd & dc.hi) | dc.magic) * inv16 + m72) * sc;
-        const f16x2 p2 = (as_f16x2((w8 & dc.lo) | dc.magic) + m1032) * sc;
-        const f16x2 p3 = (as_f16x2((w8 & dc.hi) | dc.magic) * inv16 + m72) * sc;
-        a[i][st] = __builtin_bit_cast(f16x8, u32x4{as_u32(p0), as_u32(p1), as_u32(p2), as_u32(p3)});
-      }
-    }
-    const uint8_t* xb = smem + b * kXBuf;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      f16x8 bx[4];
-#pragma unroll
-      for (int st = 0; st < 4; ++st)
-        bx[st] = *reinterpret_cast<const f16x8*>(xb + 16 * swz(16 * mt + r, 4 * q + st));
-#pragma unroll
-      for (int st = 0; st < 4; ++st)
-#pragma unroll
-        for (int i = 0; i < PT; ++i) acc[i][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i][st], bx[st], acc[i][mt], 0, 0, 0);
-    }
+  for (int st = 0; st < 4; ++st) xrd[st] = 256 * r + 16 * ((4 * q + st) ^ xswz(r));
+  auto decode = [&](int d, int i, int st) {                 // (u - 8) exact, times the scale: one rounding
+    const f16 sv = __builtin_bit_cast(f16, (uint16_t)rs[d][i]);
+    const f16x2 sc = {sv, sv};
+    const uint32_t wd = rw[d][i][st], w8 = wd >> 8;
+    const f16x2 p0 = (as_f16x2((wd & dc.lo) | dc.magic) + m1032) * sc;
+    const f16x2 p1 = (as_f16x2((wd & dc.hi) | dc.magic) * inv16 + m72) * sc;
+    const f16x2 p2 = (as_f16x2((w8 & dc.lo) | dc.magic) + m1032) * sc;
+    const f16x2 p3 = (as_f16x2((w8 & dc.hi) | dc.magic) * inv16 + m72) * sc;
+    return __builtin_bit_cast(f16x8, u32x4{as_u32(p0), as_u32(p1), as_u32(p2), as_u32(p3)});
   };
-
+  // One chunk as 4 MT / 2 groups of two activation tiles: while a group's 2 PT MFMAs run, the next group's two B fragments
+  // are read and a share of the next k-step's A fragments decoded, across the chunk's end too. Chunk j's x sits in LDS
+  // buffer j % 2, its weights in slot j % 2. The slot is refilled two chunks ahead when its last k-step has been decoded;
+  // before the last group, when every B fragment of the chunk has been read, one barrier makes the next chunk's x
+  // visible (the wait leaves the 2 PT newer weight loads in flight) and frees this chunk's buffer for the x two chunks
+  // ahead. (Left to itself hipcc waits for every pair of fragment reads right after issuing it.)
+  constexpr int GP = MT / 2, DPG = (PT + GP - 1) / GP;      // groups per k-step, decodes per group
+  f16x8 a[2][PT], bx[2][2];
+  auto chunk = [&](int j, auto slot) __attribute__((always_inline)) {
+    constexpr int d = decltype(slot)::value;
+    unrolled<4 * GP>([&](auto gi) __attribute__((always_inline)) {   // (a plain loop of this size is not unrolled)
+      constexpr int g = decltype(gi)::value, st = g / GP, mp = g % GP, nst = (g + 1) / GP % 4, nmp = (g + 1) % GP;
+      constexpr bool last = g + 1 == 4 * GP;
+      if constexpr (g == 3 * GP) issue_w(d, cb + j + 2);
+      if constexpr (last) {
+        lds_wait_barrier<2 * PT>();
+        issue_x(d, cb + j + 2);
+      }
 #pragma unroll
-  for (int e = 0; e < XL; ++e) issue_x(e, cb + e);
+      for (int e = 0; e < 2; ++e)
+        bx[(g + 1) & 1][e] =
+            *reinterpret_cast<const f16x8*>(smem + (last ? d ^ 1 : d) * kXBuf + 4096 * (2 * nmp + e) + xrd[nst]);
 #pragma unroll
-  for (int d = 0; d < D; ++d) issue_w(d, cb + d);
-  stage_x(0, 0);
-  __syncthreads();
-
-  // step j: chunk cb + j, weight slot j % D, x register set j % XL, LDS buffer j % 2. The x of chunk j + XL goes
-  // into the set chunk j used (already in LDS) before the MFMAs; after them chunk j + 1 is staged into the other
-  // buffer and the weight slot just consumed is refilled D chunks ahead. The loop is unrolled D times (D % XL == 0),
-  // so every slot and set index is a constant.
+      for (int i = DPG * mp; i < DPG * mp + DPG && i < PT; ++i) a[(st + 1) & 1][i] = decode(st == 3 ? d ^ 1 : d, i, (st + 1) & 3);
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int i = 0; i < PT; ++i)
+          acc[i][2 * mp + e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[st & 1][i], bx[g & 1][e], acc[i][2 * mp + e], 0, 0, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);    // 2 LDS reads, then 2 vector instructions to each MFMA
+#pragma unroll
+      for (int u = 0; u < 2 * PT; ++u) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 2, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  issue_w(0, cb);
+  issue_x(0, cb);
+  issue_w(1, cb + 1);
+  issue_x(1, cb + 1);
+  lds_wait_barrier<2 * PT + XP>();                          // chunk 0 of x has landed
+#pragma unroll
+  for (int e = 0; e < 2; ++e) bx[0][e] = *reinterpret_cast<const f16x8*>(smem + 4096 * e + xrd[0]);
+#pragma unroll
+  for (int i = 0; i < PT; ++i) a[0][i] = decode(0, i, 0);
   int j0 = 0;
-  for (; j0 + D <= nsteps; j0 += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int j = j0 + d;
-      if (j + XL < nsteps) issue_x(d % XL, cb + j + XL);
-      consume(d, j & 1);
-      issue_w(d, cb + j + D);
-      if (j + 1 < nsteps) stage_x((d + 1) % XL, (j + 1) & 1);
-      __syncthreads();
-    }
+  for (; j0 + 2 <= nsteps; j0 += 2) {
+    chunk(j0, std::integral_constant<int, 0>{});
+    chunk(j0 + 1, std::integral_constant<int, 1>{});
   }
-#pragma unroll
-  for (int d = 0; d < D - 1; ++d) {
-    const int j = j0 + d;
-    if (j < nsteps) {
-      if (j + XL < nsteps) issue_x(d % XL, cb + j + XL);
-      consume(d, j & 1);
-      if (j + 1 < nsteps) stage_x((d + 1) % XL, (j + 1) & 1);
-      __syncthreads();
-    }
-  }
+  if (j0 < nsteps) chunk(j0, std::integral_constant<int, 0>{});
+  vm_drain();                                               // no load into LDS is left in flight
 
-  const bool vec = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
-  auto store4 = [&](int m, int n, const f32x4& v) {
-    f16* dst = y + (size_t)m * N + n;
-    if (vec) {
-      const f16x2 lo = {epi_value(epi.mode, epi.aux, v[0], m, n, N), epi_value(epi.mode, epi.aux, v[1], m, n + 1, N)};
-      const f16x2 hi = {epi_value(epi.mode, epi.aux, v[2], m, n + 2, N), epi_value(epi.mode, epi.aux, v[3], m, n + 3, N)};
-      *reinterpret_cast<uint2*>(dst) = make_uint2(as_u32(lo), as_u32(hi));
-    } else {
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (n + e < N) dst[e] = epi_value(epi.mode, epi.aux, v[e], m, n + e, N);
-    }
-  };
-  auto store4_silu = [&](int m, int n, const f32x4& g, const f32x4& u) {
-    f16* dst = y + (size_t)m * (N / 2) + 8 * (n >> 4) + (n & 15);
-    const f16x2 lo = {silu_mul(g[0], u[0]), silu_mul(g[1], u[1])}, hi = {silu_mul(g[2], u[2]), silu_mul(g[3], u[3])};
-    *reinterpret_cast<uint2*>(dst) = make_uint2(as_u32(lo), as_u32(hi));
-  };
-  if (S == 1) {
-    if constexpr (ROPE) {                                   // per tile: the MT column tiles' loads and RoPE, then stores
-#pragma unroll
-      for (int i = 0; i < PT; ++i) {
-        Out4 out[MT];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const int m = m0 + 16 * mt + r, n = n0 + 16 * (PT * wave + i) + 4 * q;
-          const f32x4 v = acc[i][mt];                       // partner rows 8 + 4 q + v sit 32 lanes on (q + 2)
-          const f32x4 up = {shfl_down32(v[0]), shfl_down32(v[1]), shfl_down32(v[2]), shfl_down32(v[3])};
-          out[mt] = q < 2 && m < M && n < N ? rope_qkv_out4(epi, m, n, v, up) : Out4{};
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) store_rope4(out[mt]);
-      }
-      return;
-    }
+  if (S > 1) {
+    // fp32 partials of the tile, [split][fragment][thread] 16 bytes each: every store and load is one contiguous KB a wave
+    constexpr int kFrag = 16 * kThreads, kPart = PT * MT * kFrag;
+    const __amdgpu_buffer_rsrc_t pr =
+        make_rsrc(reinterpret_cast<uint8_t*>(part) + (size_t)(tile - full) * S * kPart, (uint32_t)(S * kPart));
 #pragma unroll
     for (int i = 0; i < PT; ++i)
 #pragma unroll
+      for (int mt = 0; mt < MT; ++mt) store_partial4(pr, sp * kPart + (i * MT + mt) * kFrag + 16 * tid, acc[i][mt]);
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);               // the partials' stores stay before the wait
+    __builtin_amdgcn_s_waitcnt(0);                          // every partial acknowledged: visible to all XCDs
+    __builtin_amdgcn_s_barrier();
+    int& s_last = *reinterpret_cast<int*>(smem);            // (the x buffers are free)
+    uint32_t* count = ctr + (tile - full);
+    if (tid == 0) {
+      const uint32_t prev = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_last = prev == (uint32_t)(S - 1);
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_s_barrier();
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);               // the partials' loads stay after the count
+    if (!s_last) return;
+    if (tid == 0) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the sum in split order; the loads of 8 fragments (all of them in small tiles) go out before the first add
+    constexpr int kBatch = PT * MT < 8 ? PT * MT : 8;
+#pragma unroll
+    for (int f0 = 0; f0 < PT * MT; f0 += kBatch) {
+      f32x4 sum[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) sum[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+      f32x4 v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) v[u] = load_partial4(pr, (f0 + u) * kFrag + 16 * tid);
+      for (int k = 1; k <= S; ++k) {                        // the next split's are requested before this one's are added
+        f32x4 nv[kBatch];
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u)
+          nv[u] = load_partial4(pr, k < S ? k * kPart + (f0 + u) * kFrag + 16 * tid : kOutOfRange);
+#pragma unroll
+        for (int u = 0; u < kBatch; ++u) {
+          sum[u] += v[u];
+          v[u] = nv[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) acc[(f0 + u) / MT][(f0 + u) % MT] = sum[u];
+    }
+  }
+  if constexpr (ROPE) {                                     // per tile: the MT column tiles' loads and RoPE, then stores
+#pragma unroll
+    for (int i = 0; i < PT; ++i) {
+      Out4 out[MT];
+#pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const int m = m0 + 16 * mt + r, n = n0 + 16 * (PT * wave + i) + 4 * q;
-        const f32x4 v = acc[i][mt];
-        if (epi.mode == kEpiSiluMul) {                      // up rows 8 + 4 q + v sit 32 lanes on (q + 2)
-          const f32x4 up = {shfl_down32(v[0]), shfl_down32(v[1]), shfl_down32(v[2]), shfl_down32(v[3])};
-          if (q < 2 && m < M && n < N) store4_silu(m, n, v, up);
-          continue;
-        }
-        if (m >= M || n >= N) continue;
-        store4(m, n, v);
+        const f32x4 v = acc[i][mt];                         // partner rows 8 + 4 q + v sit 32 lanes on (q + 2)
+        const f32x4 up = {shfl_down32(v[0]), shfl_down32(v[1]), shfl_down32(v[2]), shfl_down32(v[3])};
+        out[mt] = q < 2 && m < M && n < N ? rope_qkv_out4(epi, m, n, v, up) : Out4{};
       }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) store_rope4(out[mt]);
+    }
     return;
   }
-  // [S][M][N] fp32 partials, byte offsets into the workspace (S M N 4 bytes, within the 32-bit range the planner keeps)
-  const __amdgpu_buffer_rsrc_t pr = make_rsrc(part, (uint32_t)((size_t)S * M * N * 4));
-  auto poff = [&](int k, int m, int n) { return (int)((((size_t)k * M + m) * N + n) * 4); };
+  // The tile's fp16 values through LDS, so that y and the bias / residual move in 16-byte pieces of contiguous rows: a
+  // lane holds 4 rows n of one m, and storing those 8 bytes as they are makes every wave-store 16 rows of 32 bytes (at
+  // 2048 x 16384 outputs the stores alone took 35 us a round of tiles). Rows are padded by 32 bytes: the 16 rows x 32
+  // bytes of a wave's write then meet different banks.
+  const bool silu = epi.mode == kEpiSiluMul;
+  const int oc = silu ? kRows / 2 : kRows;                  // output columns of the tile
+  const int pitch = 2 * oc + 32;
+  lds_barrier();                                            // (s_last has been read)
 #pragma unroll
   for (int i = 0; i < PT; ++i)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      const int m = m0 + 16 * mt + r, n = n0 + 16 * (PT * wave + i) + 4 * q;
-      if (m >= M || n >= N) continue;
-      const int off = poff(sp, m, n);
-      if (vec) {
-        store_partial4(pr, off, acc[i][mt]);
+      const f32x4 v = acc[i][mt];
+      uint8_t* row = smem + (16 * mt + r) * pitch;
+      if (silu) {                                           // up rows 8 + 4 q + v sit 32 lanes on (q + 2)
+        const f32x4 up = {shfl_down32(v[0]), shfl_down32(v[1]), shfl_down32(v[2]), shfl_down32(v[3])};
+        const f16x2 lo = {silu_mul(v[0], up[0]), silu_mul(v[1], up[1])}, hi = {silu_mul(v[2], up[2]), silu_mul(v[3], up[3])};
+        if (q < 2) *reinterpret_cast<uint2*>(row + 16 * (PT * wave + i) + 8 * q) = make_uint2(as_u32(lo), as_u32(hi));
       } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < N) store_partial(pr, off + 4 * e, acc[i][mt][e]);
+        const f16x2 lo = {(f16)v[0], (f16)v[1]}, hi = {(f16)v[2], (f16)v[3]};
+        *reinterpret_cast<uint2*>(row + 32 * (PT * wave + i) + 8 * q) = make_uint2(as_u32(lo), as_u32(hi));
       }
     }
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);                 // the partials' stores stay before the wait
-  __builtin_amdgcn_s_waitcnt(0);                            // every partial acknowledged: visible to all XCDs
-  __builtin_amdgcn_s_barrier();
-  if (tid == 0) {
-    const uint32_t prev = __hip_atomic_fetch_add(ctr + tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    s_last = prev == (uint32_t)(S - 1);
-  }
-  __builtin_amdgcn_s_waitcnt(0);
-  __builtin_amdgcn_s_barrier();
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);                 // the partials' loads stay after the count
-  if (!s_last) return;
-  if (tid == 0) __hip_atomic_store(ctr + tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const int nrows = min(kRows, N - n0), nq = (nrows + 3) >> 2, mrows = min(16 * MT, M - m0);
-  auto split_sum = [&](int m, int n) {                      // partials of rows n .. n + 3, added in split order
-    return sum_partials4(pr, S, (N & 3) == 0 ? 4 : min(4, N - n), [&](int k) { return poff(k, m, n); });
-  };
-  for (int it = tid; it < mrows * nq; it += kThreads) {
-    const int m = m0 + it / nq, n = n0 + 4 * (it % nq);
-    if constexpr (ROPE) {
-      if ((n & 15) < 8) store_rope4(rope_qkv_out4(epi, m, n, split_sum(m, n), split_sum(m, n + 8)));
-    } else if (epi.mode == kEpiSiluMul) {
-      if ((n & 15) < 8) store4_silu(m, n, split_sum(m, n), split_sum(m, n + 8));
+  lds_barrier();
+  const int ny = silu ? N / 2 : N, c0 = silu ? n0 / 2 : n0, pcs = oc / 8;
+  const bool aux = epi.mode == kEpiBias || epi.mode == kEpiResidual;
+  const bool vec = (ny & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0 &&
+                   (!aux || (reinterpret_cast<uintptr_t>(epi.aux) & 15) == 0);
+  for (int p = tid; p < 16 * MT * pcs; p += kThreads) {
+    const int row = p / pcs, m = m0 + row, n = c0 + 8 * (p % pcs);
+    if (m >= M || n >= ny) continue;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(smem + row * pitch + 16 * (p % pcs));
+    f16* dst = y + (size_t)m * ny + n;
+    const f16* add = epi.mode == kEpiBias ? epi.aux + n : epi.aux + (size_t)m * ny + n;
+    if (vec) {
+      u32x4 o = v;
+      if (aux) {
+        const u32x4 t = *reinterpret_cast<const u32x4*>(add);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = as_u32(as_f16x2(v[e]) + as_f16x2(t[e]));
+      }
+      *reinterpret_cast<u32x4*>(dst) = o;
     } else {
-      store4(m, n, split_sum(m, n));
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n + e < ny) dst[e] = aux ? as_f16x2(v[e >> 1])[e & 1] + add[e] : as_f16x2(v[e >> 1])[e & 1];
     }
   }
 }
 
 namespace {
 
-template <int MT, int D, int NW, int XL, int PT = 4>
+template <int MT, int PT>
 hipError_t launch_prefill(const GemvArgs& a, const PrefillPlan& p, uint32_t* ctr, float* part) {
-  if constexpr (!prefill_fits(MT, D, NW, XL)) {
-    return hipErrorInvalidConfiguration;                    // never planned
-  } else {
-  const size_t shmem = (size_t)2 * 16 * MT * 256;
+  // two x buffers; the output tile of the epilogue takes their place
+  constexpr size_t shmem = std::max((size_t)2 * 16 * MT * 256, (size_t)16 * MT * (128 * PT + 32));
+  static_assert(shmem <= 65536, "above the default dynamic LDS limit");
   // the RoPE epilogue is its own instantiation: its registers would cost every other epilogue occupancy
-  auto kern = a.epi.mode == kEpiRopeQKV ? gemm_prefill<MT, D, NW, XL, PT, true> : gemm_prefill<MT, D, NW, XL, PT, false>;
-  if (shmem > 65536) {
-    static const hipError_t attr[2] = {allow_lds(gemm_prefill<MT, D, NW, XL, PT, false>, shmem),
-                                       allow_lds(gemm_prefill<MT, D, NW, XL, PT, true>, shmem)};
-    if (attr[0] != hipSuccess) return attr[0];
-    if (attr[1] != hipSuccess) return attr[1];
-  }
-  return launch(kern, dim3(p.items), dim3(64 * NW), shmem, a.stream, a.x, a.w, a.s, a.y, a.M, a.N, a.K, a.G, p.S, p.MG,
+  auto kern = a.epi.mode == kEpiRopeQKV ? gemm_prefill<MT, PT, true> : gemm_prefill<MT, PT, false>;
+  return launch(kern, dim3(p.items), dim3(256), shmem, a.stream, a.x, a.w, a.s, a.y, a.M, a.N, a.K, a.G, p.S, p.MG, p.full,
                 p.items, ctr, part, a.epi);
-  }
 }
 
-template <int MT, int NW>
-hipError_t dispatch_prefill_ring(const GemvArgs& a, const PrefillPlan& p, uint32_t* ctr, float* part) {
-  if constexpr (MT == 4 && NW == 4) {                       // fewer tiles per wave: the default shape only
-    if (p.D == 2 && p.XL == 1 && p.PT == 1) return launch_prefill<4, 2, 4, 1, 1>(a, p, ctr, part);
-    if (p.D == 2 && p.XL == 1 && p.PT == 2) return launch_prefill<4, 2, 4, 1, 2>(a, p, ctr, part);
+// The tile shapes built, and what a launch of each costs (us): `groups` workgroups share a CU (registers, LDS); `base` for
+// a launch; a workgroup takes `alone` per 128-k chunk, or a CU's resident ones `each` per chunk and workgroup when that is
+// more; a K split costs `split` and `per_mb` per MB of partials. Fitted to an MI355X sweep (graph-timed, cold weights, 65
+// to 2048 rows of 12 Qwen2.5-0.5B .. 7B projections, 1 to 8 splits; the fit's error is 10-15%); the cheapest plan by it
+// is 2.5% slower than the sweep's best on average and 26% at worst.
+struct PrefillShape {
+  int MT, PT, groups;
+  float base, alone, each, split, per_mb;
+};
+constexpr PrefillShape kPrefillShapes[] = {
+    {8, 2, 2, 4.8f, 1.20f, 0.93f, 4.4f, 0.30f},             // 128 activation rows x 128 weight rows
+    {6, 4, 2, 6.8f, 1.41f, 1.25f, 6.9f, 0.24f},             // 96 x 256
+    {4, 2, 4, 4.2f, 0.74f, 0.56f, 2.7f, 0.31f},             // 64 x 128
+    {4, 1, 4, 2.5f, 0.66f, 0.385f, 2.0f, 0.38f},            // 64 x 64
+};
+constexpr int kCUs = 256;
+
+struct PrefillCount {
+  long tiles, full, rest;
+  int S;
+};
+
+// the tiles of a shape, those that fill whole rounds, and the split of the others: at most `S`, within K and the workspace
+PrefillCount count_prefill(const PrefillShape& c, int M, int N, int KC, int S, bool all, size_t part_bytes) {
+  PrefillCount n;
+  n.tiles = (long)((M + 16 * c.MT - 1) / (16 * c.MT)) * ((N + 64 * c.PT - 1) / (64 * c.PT));
+  const long slots = (long)kCUs * c.groups;
+  n.full = all ? 0 : n.tiles / slots * slots;
+  n.rest = n.tiles - n.full;
+  n.S = std::min({S, KC, kMaxSplits});
+  const size_t tile_bytes = (size_t)16 * c.MT * 64 * c.PT * sizeof(float);   // fp32 partials of a tile
+  if (n.rest > 0) n.S = (int)std::min<size_t>((size_t)n.S, part_bytes / (tile_bytes * n.rest));
+  if (n.rest == 0 || n.rest > (long)(kCounterBytes / 4)) n.S = 1;   // one arrival counter a tile
+  if (n.S <= 1) n.S = 1, n.full = n.tiles, n.rest = 0;
+  return n;
+}
+
+float prefill_cost(const PrefillShape& c, const PrefillCount& n, int KC) {
+  const long slots = (long)kCUs * c.groups;
+  auto rounds = [&](long items) {                           // us per chunk of `items` workgroups
+    const long last = items % slots;
+    return (items / slots) * std::max(c.alone, c.groups * c.each) +
+           (last ? std::max(c.alone, ((last + kCUs - 1) / kCUs) * c.each) : 0.f);
+  };
+  float t = c.base + KC * rounds(n.full);
+  if (n.rest > 0) {
+    const float mb = (float)n.S * n.rest * (16 * c.MT * 64 * c.PT * 4) * 1e-6f;
+    t += KC * rounds(n.rest * n.S) / n.S + c.split + c.per_mb * mb;
   }
-  if (p.D == 3) return launch_prefill<MT, 3, NW, 1>(a, p, ctr, part);
-  return p.XL == 2 ? launch_prefill<MT, 2, NW, 2>(a, p, ctr, part) : launch_prefill<MT, 2, NW, 1>(a, p, ctr, part);
+  return t;
 }
 
 }  // namespace
 
-// Launch shape from an MI355X sweep (graph-timed, M = 128 / 256 / 512 / 2048 on the Qwen2.5-3B and 7B projections):
-// 64 activation rows x 4 waves with a 2-deep weight ring (2 workgroups per CU; deeper rings or the x lookahead cost
-// the second wave per SIMD and lose), 4, 2 or 1 weight tiles per wave (below); K split into the largest power of two
-// that keeps >= 16 chunks per split and at most two rounds of kPrefillTargetGroups workgroups, within the workspace
-// and the counters. The tuning override selects (waves_per_group: 1 = MT 4 / 4 waves, 2 = MT 4 / 8 waves, 4 = MT 8 /
-// 4 waves, 8 = MT 8 / 8 waves; ring: 2 or 3 = weight chunks in flight, 4 = two in flight with a two-chunk x lookahead),
-// always with 4 tiles per wave.
+// Launch shape: the cheapest of the tile shapes and of 1, 2, 3, 4, 6, 8 splits (at least 4 chunks each) of the tiles that
+// do not fill a round. The tuning override selects the shape (waves_per_group: 1 or 2 = 64 x 128, 4 or 8 = 128 x 128) and
+// the split of all tiles (k_splits).
 PrefillPlan plan_gemm_prefill(int M, int N, int K, size_t workspace_bytes) {
-  PrefillPlan p;
   const GemvOverride o = gemv_override();
   const int KC = K / 128;
-  switch (o.waves) {
-    case 1: p.MT = 4; p.NW = 4; break;
-    case 2: p.MT = 4; p.NW = 8; break;
-    case 4: p.MT = 8; p.NW = 4; break;
-    case 8: p.MT = 8; p.NW = 8; break;
-    default: p.MT = 4; p.NW = 4; break;
+  const size_t part_bytes = workspace_bytes > kCounterBytes ? workspace_bytes - kCounterBytes : 0;
+  PrefillPlan p;
+  float best = -1.f;
+  for (const PrefillShape& c : kPrefillShapes) {
+    if (o.waves > 0 && (c.PT != 2 || c.MT != (o.waves >= 4 ? 8 : 4))) continue;
+    for (int S : {1, 2, 3, 4, 6, 8}) {
+      if (o.splits > 0 ? S != 1 : S > 1 && KC < 4 * S) continue;
+      const PrefillCount n = count_prefill(c, M, N, KC, o.splits > 0 ? o.splits : S, o.splits > 0, part_bytes);
+      const float t = prefill_cost(c, n, KC);
+      if (best >= 0.f && t >= best) continue;
+      best = t;
+      p.MT = c.MT;
+      p.PT = c.PT;
+      p.MG = (M + 16 * c.MT - 1) / (16 * c.MT);
+      p.S = n.S;
+      p.full = (int)n.full;
+      p.items = (int)(n.full + n.rest * n.S);
+    }
   }
-  p.D = o.ring == 3 ? 3 : 2;
-  p.XL = o.ring == 4 ? 2 : 1;
-  if (!prefill_fits(p.MT, p.D, p.NW, p.XL)) p.NW = 4;      // 8 waves: 256 registers per wave, D = 2 and MT = 4 only
-  if (!prefill_fits(p.MT, p.D, p.NW, p.XL)) p.D = 2;
-  p.MG = (M + 16 * p.MT - 1) / (16 * p.MT);
-  // fewer 16-row tiles per wave (default shape only): 2 up to 8 activation tiles (168 instead of 256 registers, a third
-  // wave per SIMD: 3B merged gate|up at M = 512 89 -> 77 us, 7B gate|up 133 -> 106; at M = 2048 4 tiles stay ahead,
-  // 365 vs 388), then halved while the grid holds less than two workgroups per CU. A wave's activation bytes per
-  // chunk stay the same while its weight bytes shrink (x : w = 4 : PT), so past 4 activation tiles a long K (>= 128
-  // chunks) splits across workgroups instead (7B down, M = 512: 130 us at 4 tiles and 2 splits vs 142 at 1 tile;
-  // M = 2048: 351 vs 451; at M <= 256 and on K <= 11008 the thin tiles win up to 2.9x)
-  auto groups = [&](int pt) { return (long)((N + 16 * pt * p.NW - 1) / (16 * pt * p.NW)) * p.MG; };
-  p.PT = 4;
-  if (o.waves == 0 && o.ring == 0 && (KC < 128 || p.MG <= 4)) {
-    if (p.MG <= 8) p.PT = 2;
-    while (p.PT > 1 && groups(p.PT) < 2 * kPrefillTargetGroups) p.PT /= 2;
-  }
-  const long tiles = groups(p.PT);
-  // the partials are addressed with 32-bit byte offsets (a buffer resource): at most 2^31 - 1 bytes of them
-  const size_t part_bytes = std::min<size_t>(workspace_bytes > kCounterBytes ? workspace_bytes - kCounterBytes : 0,
-                                             (size_t)INT_MAX);
-  int S = 1;
-  if (o.splits > 0) {
-    S = o.splits;
-  } else if (part_bytes > 0) {
-    while (S < kMaxSplits && tiles * 2 * S <= 2 * kPrefillTargetGroups && KC >= 16 * 2 * S) S *= 2;
-  }
-  S = std::min(S, std::max(1, KC));
-  while (S > 1 && (size_t)S * M * N * sizeof(float) > part_bytes) --S;
-  if (tiles > (long)(kCounterBytes / 4)) S = 1;
-  p.S = std::max(S, 1);
-  p.items = (int)(tiles * p.S);
   return p;
 }
 
@@ -377,8 +431,9 @@ hipError_t gemm_prefill_launch(const GemvArgs& a, void* workspace, size_t worksp
   const PrefillPlan p = plan_gemm_prefill(a.M, a.N, a.K, workspace ? workspace_bytes : 0);
   uint32_t* ctr = static_cast<uint32_t*>(workspace);
   float* part = workspace ? reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + kCounterBytes) : nullptr;
-  if (p.MT == 4) return p.NW == 8 ? dispatch_prefill_ring<4, 8>(a, p, ctr, part) : dispatch_prefill_ring<4, 4>(a, p, ctr, part);
-  return p.NW == 8 ? dispatch_prefill_ring<8, 8>(a, p, ctr, part) : dispatch_prefill_ring<8, 4>(a, p, ctr, part);
+  if (p.MT == 8) return launch_prefill<8, 2>(a, p, ctr, part);
+  if (p.MT == 6) return launch_prefill<6, 4>(a, p, ctr, part);
+  return p.PT == 2 ? launch_prefill<4, 2>(a, p, ctr, part) : launch_prefill<4, 1>(a, p, ctr, part);
 }
 
 }  // namespace lowbit

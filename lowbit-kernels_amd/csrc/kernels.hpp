@@ -212,14 +212,12 @@ struct GemvPlan {
 
 // launch shape of the prefill GEMM (M > 64)
 struct PrefillPlan {
-  int MT = 8;       // 16-row activation tiles per workgroup
-  int D = 2;        // weight chunks in flight per wave
-  int S = 1;        // workgroups splitting K per tile
+  int MT = 4;       // 16-row activation tiles per workgroup
+  int PT = 1;       // 16-row weight tiles per wave (4 waves)
   int MG = 1;       // activation-row groups
-  int items = 1;    // workgroups: tiles x S
-  int NW = 4;       // waves per workgroup, 16 PT weight rows each
-  int XL = 1;       // chunks of x in flight
-  int PT = 4;       // 16-row weight tiles per wave
+  int S = 1;        // workgroups splitting K per tile past the first `full` tiles, which take one each
+  int full = 0;
+  int items = 1;    // workgroups: full + S x the other tiles
 };
 
 // process-wide launch-shape override for tuning sweeps (lowbit_set_launch_override); 0 = automatic
@@ -266,8 +264,6 @@ constexpr size_t kLdsPerCu = 160 * 1024;  // gfx950
 constexpr int kGemmMaxGroups = 256;
 constexpr int kGemmTargetWaves = 1792;
 constexpr int kGemmMaxWavesWide = 2048;
-// prefill GEMM: K is split while the work items fill fewer than two rounds of this many workgroups
-constexpr int kPrefillTargetGroups = 256;
 // decode attention: when the cache holds at least kAttnMinSplitKeys keys, keys are split across blocks while
 // (token, head group) blocks number fewer than kAttnTargetBlocks, down to kAttnMinKeys keys per block
 constexpr int kAttnTargetBlocks = 256;
@@ -328,11 +324,6 @@ hipError_t gemv_rowmajor_launch(const GemvArgs& a, int rows_per_wave, bool v3);
 hipError_t gemv_f16w_launch(const GemvArgs& a);
 hipError_t gemm_mfma_launch(const GemvArgs& a, int row_tiles, void* workspace, size_t workspace_bytes);
 hipError_t zero_words_launch(void* p, int n, hipStream_t stream);
-// prefill variants that compile without register spills (hipcc -O3, gfx950): an 8-wave workgroup has 256 registers
-// per wave, enough for 4 activation tiles and a 2-deep weight ring only
-constexpr bool prefill_fits(int MT, int D, int NW, int XL) {
-  return (D == 2 || XL == 1) && (NW == 4 || (MT == 4 && D == 2));
-}
 PrefillPlan plan_gemm_prefill(int M, int N, int K, size_t workspace_bytes);
 hipError_t gemm_prefill_launch(const GemvArgs& a, void* workspace, size_t workspace_bytes);
 hipError_t rmsnorm_launch(const f16* x, const f16* w, f16* out, int M, int H, float eps, hipStream_t st);

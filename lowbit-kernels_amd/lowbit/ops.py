@@ -161,15 +161,22 @@ def dequant(wq, layout=None):
 AUTO_GEMV_ROWS, AUTO_V5_ROWS, AUTO_V5_WIDE_ROWS, AUTO_WIDE_N = 1, 64, 64, 3072
 AUTO_GEMV_NARROW_ROWS, AUTO_GEMV_NARROW_N, AUTO_GEMV_MAX_K = 3, 8192, 16384
 # Beyond the MFMA kernel's rows (prefill), a weight on the mma layout goes to the int4-direct prefill GEMM (prefill())
-# when K >= AUTO_PREFILL_MIN_K, when M <= AUTO_PREFILL_ROWS, or when M <= AUTO_PREFILL_NARROW_ROWS on a small layer
-# (N and K <= AUTO_PREFILL_NARROW); everything else dequantizes (4.4-4.8 TB/s) and calls BLAS. From the MI355X sweep at
-# M = 128, 256, 512, 2048 on the Qwen2.5-3B / 7B projections (int4 vs dequantize + hipBLASLt, us): every layer up to
-# 512 rows (3B merged gate|up 26.3 vs 45.9 at 128, 72.6 vs 75.9 at 512; 3B down 26.0 vs 38.3 at 128, 49.0 vs 58.4 at
-# 512; 7B gate|up 97.8 vs 100.8 at 512), the attention-sized 3B layers up to 2048 rows (o 29.2 vs 31.7, q|k|v 36.9 vs
-# 36.6 at 2048) and the long-K 7B down at every M (47 vs 109 at 128, 119 vs 203 at 512, 345 vs 395 at 2048);
-# dequantize + hipBLASLt keeps the wide and long layers at 2048 rows (3B gate|up 190 vs 261, 3B down 107 vs 134).
+# when K >= AUTO_PREFILL_MIN_K, up to AUTO_PREFILL_ROWS rows, up to AUTO_PREFILL_WIDE_ROWS rows on a narrow or wide layer
+# (N <= AUTO_PREFILL_NARROW or N > AUTO_PREFILL_WIDE_N), up to AUTO_PREFILL_NARROW_ROWS rows on a small one (N and K <=
+# AUTO_PREFILL_NARROW), and up to as many where the BLAS GEMM's 256 x 256 tiles, more than one round of the 256 CUs, would
+# fill its rounds to less than AUTO_PREFILL_FILL; everything else dequantizes (4.4-4.8 TB/s) and calls BLAS. From an
+# MI355X sweep of 65 .. 2048 rows on 12 Qwen2.5-0.5B .. 7B projections (int4 vs dequantize + hipBLASLt, us): every layer
+# up to 1000 rows (2048 x 22016 20 vs 42 at 128, 56 vs 73 at 512, 96 vs 114 at 1000; 3584 x 18944 29 vs 63, 76 vs 99, 149
+# vs 164; 11008 x 2048 19 vs 35, 37 vs 54, 62 vs 73; layers of 4096 < N <= 8192, of which the sweep has one, keep the
+# older 512); the small layers at 2048 (2048 x 2048 25 vs 31, 3584 x 3584 57 vs 59) and the long-K 7B down at every M (279
+# vs 396 at 2048). At 1400 and 2048 rows the fill decides: 0.67 .. 0.77 of the rounds 2048 x 22016 at 1400 133 vs 145,
+# 3584 x 18944 at 2048 282 vs 341, 1536 x 17920 at 2048 123 vs 134; 0.86 .. 0.9 3584 x 18944 at 1400 196 vs 187, 2048 x
+# 22016 at 2048 200 vs 188; 1.0 3584 x 16384 at 2048 245 vs 205; under one round (narrow layers, where BLAS takes smaller
+# tiles) 11008 x 2048 at 2048 110 vs 104, 8960 x 1536 73 vs 72.
 AUTO_PREFILL_MIN_K, AUTO_PREFILL_ROWS = 16384, 512
+AUTO_PREFILL_WIDE_N, AUTO_PREFILL_WIDE_ROWS = 8192, 1024
 AUTO_PREFILL_NARROW, AUTO_PREFILL_NARROW_ROWS = 4096, 2048
+AUTO_PREFILL_FILL = 0.8
 
 
 def gemm_chunked(x, wq, chunk=64):
@@ -201,15 +208,23 @@ def prefill_path(m, wq):
     """True when linear() sends m rows to the int4 prefill GEMM rather than dequantize + BLAS (auto routing only)."""
     if auto_version(m, wq) is not None or wq.packed_mma is None:
         return False
-    return (wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS
-            or (m <= AUTO_PREFILL_NARROW_ROWS and wq.n <= AUTO_PREFILL_NARROW and wq.k <= AUTO_PREFILL_NARROW))
+    if wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS:
+        return True
+    if m > AUTO_PREFILL_NARROW_ROWS:
+        return False
+    narrow = wq.n <= AUTO_PREFILL_NARROW
+    if narrow and wq.k <= AUTO_PREFILL_NARROW:
+        return True
+    if m <= AUTO_PREFILL_WIDE_ROWS and (narrow or wq.n > AUTO_PREFILL_WIDE_N):
+        return True
+    tiles = -(-m // 256) * -(-wq.n // 256)
+    return tiles > 256 and tiles < AUTO_PREFILL_FILL * 256 * -(-tiles // 256)
 
 
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     """Decode (few rows): an INT4 kernel (v6 GEMV for one row, v5 MFMA beyond). Prefill (many rows): dequantize, then
     the fp16 BLAS GEMM (hipBLASLt under PyTorch-ROCm), or the int4 prefill GEMM where prefill_path says (K >=
-    AUTO_PREFILL_MIN_K at any M, every layer up to AUTO_PREFILL_ROWS rows, layers with N and K <= AUTO_PREFILL_NARROW
-    up to AUTO_PREFILL_NARROW_ROWS rows). version 0 = auto; a fixed version runs up to min(max_gemv_rows, its row
+    AUTO_PREFILL_MIN_K at any M, every layer up to AUTO_PREFILL_ROWS rows, some up to AUTO_PREFILL_NARROW_ROWS). version 0 = auto; a fixed version runs up to min(max_gemv_rows, its row
     limit) rows (v5: 64), and dequantize + BLAS above.
     bias ([N], optional; not in the reference's signature; used in fp16 on x's device on every route): y =
     fp16(x W^T) + bias in fp16, the rounding of the reference's linear() followed by `+ bias`; the v5, one-row v6 and prefill kernels add it in their store (no extra

@@ -1,0 +1,61 @@
+"""The prefill GEMM at the edges of its tile shapes (64, 96 and 128 activation rows; 64, 128 and 256 weight rows), its K
+splits and its output path (16-byte pieces, or element by element for widths and addresses that do not allow them),
+against the fp64 product of the exactly dequantized weights; and the routes above AUTO_PREFILL_ROWS rows.
+
+Bound (assert_rounds): half an fp16 ulp plus 2^-16 of the outputs' RMS for the fp32 sums."""
+import pytest
+import torch
+
+from lowbit import _native, ops
+from test_gpu_kernels import make_weight
+from test_gpu_prefill import assert_rounds, prefill
+
+pytestmark = pytest.mark.gpu
+
+
+# rows at, before and after a multiple of 64, 96 and 128; N at and off multiples of 256, 64, 16, 8, 4 and 2; one chunk of
+# K, an odd count, and long K (splits); shapes whose tiles fill one round and part of a second (whole and split tiles)
+@pytest.mark.parametrize("m,k,n", [
+    (64, 128, 64), (65, 128, 250), (95, 384, 257), (96, 640, 1000), (97, 256, 1004), (127, 1152, 998), (128, 896, 4864),
+    (129, 2048, 2050), (191, 11008, 130), (192, 8960, 1536), (193, 4096, 72), (255, 1536, 8961), (257, 128, 8960),
+    (700, 2048, 2560), (385, 1024, 11008), (1025, 640, 4099), (640, 384, 22016)])
+def test_tile_edges(cuda, m, k, n):
+    wq, *_, gen = make_weight(k, n, m + k + n, layouts=("mma",), sd=0.02)
+    x = torch.randn(m, k, generator=gen).half().cuda()
+    w = ops.dequant(wq, "mma").double()
+    y = prefill(x, wq)
+    assert_rounds(y, x.double() @ w.t())
+    assert torch.equal(prefill(x, wq), y)
+    bias = torch.randn(n, generator=gen).half().cuda()
+    assert torch.equal(prefill(x, wq, _native.EPI_BIAS, bias), y + bias)
+    res = torch.randn(m, n, generator=gen).half().cuda()
+    want = res + y
+    prefill(x, wq, _native.EPI_RESIDUAL, res, out=res)
+    assert torch.equal(res, want)
+
+
+def test_output_at_any_address(cuda):
+    wq, *_, gen = make_weight(512, 768, 3, layouts=("mma",), sd=0.02)
+    x = torch.randn(200, 512, generator=gen).half().cuda()
+    y = prefill(x, wq)
+    for off in (1, 2, 4):                                   # 2-, 4- and 8-byte aligned outputs and residuals
+        buf = torch.zeros(200 * 768 + 2 * off, dtype=torch.float16, device="cuda")
+        out = buf[off:off + 200 * 768].view(200, 768)
+        assert torch.equal(prefill(x, wq, out=out), y)
+        assert int(torch.count_nonzero(buf[:off])) == 0 and int(torch.count_nonzero(buf[off + 200 * 768:])) == 0
+        res = torch.randn(200, 768, generator=gen).half().cuda()
+        out.copy_(res)
+        assert torch.equal(prefill(x, wq, _native.EPI_RESIDUAL, out, out=out), res + y)
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 256, 8192), (513, 256, 8192), (1024, 2048, 11008), (1025, 256, 1536), (1100, 256, 17920), (1300, 256, 13000), (2048, 256, 11008),
+                                   (2048, 2048, 2560), (2049, 256, 2048)])
+def test_linear_agrees_on_both_prefill_routes(cuda, m, k, n):
+    """linear() on either side of the routing rule equals the product of the dequantized weights, with and without a
+    bias, whichever GEMM it takes."""
+    wq, *_, gen = make_weight(k, n, m + n, layouts=("mma",), sd=0.02)
+    x = torch.randn(m, k, generator=gen).half().cuda()
+    bias = torch.randn(n, generator=gen).half().cuda()
+    y = ops.linear(x, wq)
+    assert_rounds(y, x.double() @ ops.dequant(wq, "mma").double().t())
+    assert torch.equal(ops.linear(x, wq, bias=bias), y + bias)
