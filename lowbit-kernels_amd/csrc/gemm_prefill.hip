@@ -286,36 +286,52 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   // lane holds 4 rows n of one m, and storing those 8 bytes as they are makes every wave-store 16 rows of 32 bytes (at
   // 2048 x 16384 outputs the stores alone took 35 us a round of tiles). Rows are padded by 32 bytes: the 16 rows x 32
   // bytes of a wave's write then meet different banks.
-  const bool silu = epi.mode == kEpiSiluMul;
-  const int oc = silu ? kRows / 2 : kRows;                  // output columns of the tile
-  const int pitch = 2 * oc + 32;
+  constexpr int kPitch = 2 * kRows + 32;
   lds_barrier();                                            // (s_last has been read)
 #pragma unroll
   for (int i = 0; i < PT; ++i)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const f32x4 v = acc[i][mt];
-      uint8_t* row = smem + (16 * mt + r) * pitch;
-      if (silu) {                                           // up rows 8 + 4 q + v sit 32 lanes on (q + 2)
-        const f32x4 up = {shfl_down32(v[0]), shfl_down32(v[1]), shfl_down32(v[2]), shfl_down32(v[3])};
-        const f16x2 lo = {silu_mul(v[0], up[0]), silu_mul(v[1], up[1])}, hi = {silu_mul(v[2], up[2]), silu_mul(v[3], up[3])};
-        if (q < 2) *reinterpret_cast<uint2*>(row + 16 * (PT * wave + i) + 8 * q) = make_uint2(as_u32(lo), as_u32(hi));
-      } else {
-        const f16x2 lo = {(f16)v[0], (f16)v[1]}, hi = {(f16)v[2], (f16)v[3]};
-        *reinterpret_cast<uint2*>(row + 32 * (PT * wave + i) + 8 * q) = make_uint2(as_u32(lo), as_u32(hi));
-      }
+      const f16x2 lo = {(f16)v[0], (f16)v[1]}, hi = {(f16)v[2], (f16)v[3]};
+      *reinterpret_cast<uint2*>(smem + (16 * mt + r) * kPitch + 32 * (PT * wave + i) + 8 * q) = make_uint2(as_u32(lo), as_u32(hi));
     }
   lds_barrier();
-  const int ny = silu ? N / 2 : N, c0 = silu ? n0 / 2 : n0, pcs = oc / 8;
+  if (epi.mode == kEpiSiluMul) {                            // 8 outputs from a 16-row tile's 8 gate and 8 up values (all
+    constexpr int kPcs = kRows / 16;                        // lanes busy: in the registers' layout half of them hold up)
+    const int ny = N / 2;                                   // (N % 16 == 0)
+    const bool vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+    for (int p = tid; p < 16 * MT * kPcs; p += kThreads) {
+      const int row = p / kPcs, m = m0 + row, n = n0 / 2 + 8 * (p % kPcs);
+      if (m >= M || n >= ny) continue;
+      const u32x4* src = reinterpret_cast<const u32x4*>(smem + row * kPitch + 32 * (p % kPcs));
+      const u32x4 gv = src[0], uv = src[1];
+      u32x4 o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f16x2 g2 = as_f16x2(gv[e]), u2 = as_f16x2(uv[e]);
+        o[e] = as_u32(f16x2{silu_mul((float)g2[0], (float)u2[0]), silu_mul((float)g2[1], (float)u2[1])});
+      }
+      f16* dst = y + (size_t)m * ny + n;
+      if (vec) {
+        *reinterpret_cast<u32x4*>(dst) = o;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) dst[e] = as_f16x2(o[e >> 1])[e & 1];
+      }
+    }
+    return;
+  }
+  constexpr int kPcs = kRows / 8;
   const bool aux = epi.mode == kEpiBias || epi.mode == kEpiResidual;
-  const bool vec = (ny & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0 &&
+  const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0 &&
                    (!aux || (reinterpret_cast<uintptr_t>(epi.aux) & 15) == 0);
-  for (int p = tid; p < 16 * MT * pcs; p += kThreads) {
-    const int row = p / pcs, m = m0 + row, n = c0 + 8 * (p % pcs);
-    if (m >= M || n >= ny) continue;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(smem + row * pitch + 16 * (p % pcs));
-    f16* dst = y + (size_t)m * ny + n;
-    const f16* add = epi.mode == kEpiBias ? epi.aux + n : epi.aux + (size_t)m * ny + n;
+  for (int p = tid; p < 16 * MT * kPcs; p += kThreads) {
+    const int row = p / kPcs, m = m0 + row, n = n0 + 8 * (p % kPcs);
+    if (m >= M || n >= N) continue;
+    const u32x4 v = *reinterpret_cast<const u32x4*>(smem + row * kPitch + 16 * (p % kPcs));
+    f16* dst = y + (size_t)m * N + n;
+    const f16* add = epi.mode == kEpiBias ? epi.aux + n : epi.aux + (size_t)m * N + n;
     if (vec) {
       u32x4 o = v;
       if (aux) {
@@ -327,7 +343,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
-        if (n + e < ny) dst[e] = aux ? as_f16x2(v[e >> 1])[e & 1] + add[e] : as_f16x2(v[e >> 1])[e & 1];
+        if (n + e < N) dst[e] = aux ? as_f16x2(v[e >> 1])[e & 1] + add[e] : as_f16x2(v[e >> 1])[e & 1];
     }
   }
 }
