@@ -263,7 +263,9 @@ int lowbit_attention(const void* q, const void* k_cache, const void* v_cache, co
  * attention keeps at most 8 key partitions and leaves their partial softmax sums in the workspace; the projection's
  * prologue merges them into its x in partition order, the attention's own merge, so y has the bits of lowbit_attention
  * (with a workspace that holds at most the same partitions) followed by lowbit_w4_linear_fused / lowbit_f16_linear_fused
- * at M = 1 -- one launch fewer, and the attention output never written. Hq <= 32, Hq / Hkv in {1, 2, 4, 6, 7, 8};
+ * at M = 1 -- one launch fewer, and the attention output never written. On a long cache (Hq * max_keys >= 128000 and a
+ * workspace of 16 partitions or more) the attention splits the keys further and merges them itself, as lowbit_attention
+ * does there: three launches, the bits of lowbit_attention with a workspace smaller by Hq * 256 bytes. Hq <= 32, Hq / Hkv in {1, 2, 4, 6, 7, 8};
  * workspace required: 16-byte aligned, at least 4096 + Hq * 132 * 4 bytes, no initial contents (the partials, P x Hq
  * x 132 x 4 bytes, follow its first 4096). No counterpart in the reference (its decoder runs torch attention, then
  * W4Linear); it serves the fused decoder's one-token step. */

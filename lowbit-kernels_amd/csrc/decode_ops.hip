@@ -276,6 +276,44 @@ __global__ __launch_bounds__(256) void attention_combine(const float* __restrict
       (f16)merge_partitions(pr, b * P * G * kAttnRec + g * kAttnRec, G * kAttnRec, P, d);
 }
 
+// attention_combine for up to kAttnManyParts partitions: one block per (token, head), a thread per dim; the partitions'
+// weights exp(max - overall max) are evaluated once, a thread each, and shared through LDS (attention_combine has every
+// thread evaluate them all, which its at most 16 partitions hide behind one round trip)
+__global__ __launch_bounds__(kHeadDim) void attention_combine_many(const float* __restrict__ part, f16* __restrict__ out,
+                                                                   int Hq, int Hkv, int P) {
+  __shared__ float s_max[kAttnManyParts], s_f[kAttnManyParts], s_sum[kAttnManyParts];
+  const int m = blockIdx.x / Hq, hd = blockIdx.x % Hq, G = Hq / Hkv, d = threadIdx.x;
+  const float* rec = part + ((size_t)(m * Hkv + hd / G) * P * G + hd % G) * kAttnRec;   // partition p: + p G records
+  const int step = G * kAttnRec;
+  float ps = 0.f;
+  if (d < P) {
+    s_max[d] = rec[(size_t)d * step];
+    ps = rec[(size_t)d * step + 1];
+  }
+  __syncthreads();
+  float gm = -INFINITY;
+  for (int p = 0; p < P; ++p) gm = fmaxf(gm, s_max[p]);
+  if (d < P) {
+    const float f = s_max[d] == -INFINITY ? 0.f : expf(s_max[d] - gm);   // (a partition that saw no key)
+    s_f[d] = f;
+    s_sum[d] = f * ps;
+  }
+  __syncthreads();
+  float num = 0.f, den = 0.f;
+  for (int p0 = 0; p0 < P; p0 += 16) {                       // 16 loads in flight
+    float v[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = p0 + u < P ? rec[(size_t)(p0 + u) * step + 4 + d] : 0.f;
+#pragma unroll
+    for (int u = 0; u < 16; ++u)
+      if (p0 + u < P) {
+        num = fmaf(s_f[p0 + u], v[u], num);
+        den += s_sum[p0 + u];
+      }
+  }
+  out[(size_t)blockIdx.x * kHeadDim + d] = (f16)(num / den);
+}
+
 // Causal GQA attention on MFMA for multi-token steps and prompts (same contract as attention_kernel): one wave per
 // (KV head, 16 query rows, key partition), the query rows of a KV head numbered row = token * G + head-in-group.
 // Per block of 32 keys (v_mfma_f32_16x16x32_f16):
@@ -1040,34 +1078,59 @@ hipError_t launch_attention_mfma(const f16* q, const f16* k, const f16* v, const
   return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
                 Hq);
 }
-// prompts: one workgroup per (KV head, 32 RG query rows, key partition); partitions while the workgroups number fewer
-// than kAttnPromptTargetGroups, at most one per kAttnPromptMinKeys of max_keys, within the workspace
+// prompts and long caches: one workgroup per (KV head, 32 RG query rows, key partition); partitions while the workgroups
+// number fewer than `target`, at most one per kAttnPromptMinKeys of max_keys, within the workspace (a workgroup splits the
+// keys its rows actually attend, so a bound well above the real count costs only empty partitions)
 template <int RG, int KG>
 hipError_t launch_attention_prompt(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M,
                                    int Hq, int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes,
-                                   hipStream_t st) {
+                                   hipStream_t st, long target) {
   const int G = Hq / Hkv;
   const int tiles = (int)(((long)M * G + 32 * RG - 1) / (32 * RG));
   const long wgs = (long)tiles * Hkv;
   int P = 1;
-  if (ws && ws_bytes > kAttnCounterBytes && wgs < kAttnPromptTargetGroups && max_keys >= 2 * kAttnPromptMinKeys) {
-    P = (int)std::min<long>({(kAttnPromptTargetGroups + wgs - 1) / wgs,
-                             (max_keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys, (long)kAttnMaxParts});
+  if (ws && ws_bytes > kAttnCounterBytes && wgs < target && max_keys >= 2 * kAttnPromptMinKeys) {
+    P = (int)std::min<long>({(target + wgs - 1) / wgs, (max_keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys,
+                             (long)kAttnManyParts});
     const size_t per = (size_t)M * Hq * kAttnRec * sizeof(float);
     P = (int)std::max<size_t>(1, std::min<size_t>((size_t)P, (ws_bytes - kAttnCounterBytes) / per));
   }
   float* part = ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kAttnCounterBytes) : nullptr;
-  const size_t lds = std::max<size_t>((size_t)2 * 2 * 32 * KG * kHeadDim * 2, (size_t)(KG - 1) * RG * 66 * 256);
+  constexpr size_t lds = std::max<size_t>((size_t)2 * 2 * 32 * KG * kHeadDim * 2, (size_t)(KG - 1) * RG * 66 * 256);
   if (lds > 65536) {
     static const hipError_t attr = allow_lds(attention_prompt<RG, KG>, lds);
     if (attr != hipSuccess) return attr;
   }
-  hipError_t e = launch(attention_prompt<RG, KG>, dim3((unsigned)wgs, P), dim3(256), lds, st, q, k, v, pos, out, M, Hq,
-                        Hkv, L, scale, tiles, part);
+  hipError_t e = launch(attention_prompt<RG, KG>, dim3((unsigned)wgs, P), dim3(256), lds, st, q, k, v, pos, out, M, Hq, Hkv,
+                        L, scale, tiles, part);
   if (e != hipSuccess || P == 1) return e;
+  if (P > kAttnMaxParts)
+    return launch(attention_combine_many, dim3((unsigned)(M * Hq)), dim3(kHeadDim), 0, st, part, out, Hq, Hkv, P);
   const long threads = (long)M * Hq * kHeadDim;
   return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
                 Hq);
+}
+// Long caches: few query rows over many keys go to the prompt kernel with the keys split over the chip, where the decode
+// kernel has every query head read K and V on its own (Hq / Hkv times) and attention_mfma's waves load theirs unshared,
+// both at most 16 ways. Its longer prologue and the merge of up to 64 partitions cost ~11 us at any length, so it starts
+// where the others pass that: 2048 keys, and M Hq keys from 80 K (one token: 128 K, since the others can leave the merge to
+// the o projection). MI355X, us (others -> this): one token, 28 / 4 heads, 3000 keys 16.7 -> 12.1, 16000 45 -> 19, 24000 64 -> 21
+// (12 / 2 heads 6000 13.3 -> 13.9, 12000 18.3 -> 16.5, 24000 28 -> 19); 4 tokens of 16 / 2 heads on 6000 23.4 -> 14.7;
+// 16 on 3000 16.1 -> 14.1 (1500: 11.2 against 11.9), 24000 72 -> 24. `max_keys` is the caller's bound; the partitions
+// follow the real count. A workspace of fewer than 16 partitions keeps the other kernels.
+bool long_attention(int M, int Hq, int Hkv, int max_keys, size_t ws_bytes) {
+  const long rows = (long)M * (Hq / Hkv);
+  if (rows >= kAttnPromptMinRows || max_keys < kAttnLongKeys) return false;
+  if ((long)M * Hq * max_keys < (M == 1 ? kAttnLongWorkOne : kAttnLongWork)) return false;
+  return ws_bytes >= kAttnCounterBytes + (size_t)16 * M * Hq * kAttnRec * sizeof(float);
+}
+hipError_t launch_attention_long(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
+                                 int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
+  // 64 rows a workgroup up to 128 rows, 32 beyond (28 / 4 heads, 32 tokens on 24000: 43 us against 53; 16 / 2, 16 on 24000:
+  // 24 against 27)
+  if ((long)M * (Hq / Hkv) <= 128)
+    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256);
+  return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256);
 }
 }  // namespace
 
@@ -1076,10 +1139,12 @@ hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int6
   const long rows = (long)M * (Hq / Hkv);
   // the prompt kernel's longer prologue and merge pay from about 384 rows (16 / 2 heads, 48 tokens on 600 cached: level
   // at 12.9 us; 28 / 4 heads, 64 on 1000: 21.7 -> 17.1; below: 16 tokens on 512 cached 9.0 against 11.4 us)
+  if (long_attention(M, Hq, Hkv, max_keys, ws ? ws_bytes : 0))
+    return launch_attention_long(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
   if (rows >= kAttnPromptMinRows) {
     if ((rows + 63) / 64 * Hkv < kAttnPromptWide && max_keys >= kAttnPromptLongKeys)
-      return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
-    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+      return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512);
+    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512);
   }
   if (rows >= kAttnMfmaMinRows)
     return launch_attention_mfma(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
@@ -1101,6 +1166,13 @@ hipError_t attention_partials_launch(const f16* q, const f16* k, const f16* v, c
                                      hipStream_t st) {
   // one token: the decode kernel with one query head per block (the MFMA kernel takes 32 or more rows per KV head)
   if (Hq / Hkv >= kAttnMfmaMinRows || Hkv >= 64) return hipErrorInvalidValue;
+  // a long cache: merged here, into out; the partials then start behind out in the workspace (out [Hq * 128] is its start)
+  const size_t xbytes = (size_t)Hq * kHeadDim * sizeof(f16);
+  if (ws_bytes > xbytes && long_attention(1, Hq, Hkv, max_keys, ws_bytes - xbytes)) {
+    *parts = 1;
+    return launch_attention_long(q, k, v, pos, out, 1, Hq, Hkv, L, max_keys, scale, static_cast<uint8_t*>(ws) + xbytes,
+                                 ws_bytes - xbytes, st);
+  }
   return launch_attention<1, 32>(q, k, v, pos, out, 1, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, kAttnXMaxParts,
                                  false, parts);
 }

@@ -288,7 +288,10 @@ constexpr int kAttnMfmaTargetWaves = 512;
 constexpr int kAttnPromptMinRows = 384;
 constexpr int kAttnPromptWide = 160;
 constexpr int kAttnPromptLongKeys = 1024;
-constexpr int kAttnPromptTargetGroups = 512;
+constexpr int kAttnManyParts = 64;        // its key partitions at most
+// fewer rows go there too from kAttnLongKeys keys and this many (token, head, key)s
+constexpr int kAttnLongKeys = 2048;
+constexpr long kAttnLongWork = 80000, kAttnLongWorkOne = 128000;
 constexpr int kAttnPromptMinKeys = 128;
 constexpr int kAttnManyBlocks = 512;      // from this many blocks on, at most 4 waves per block
 constexpr int kMaxSplits = 32;
@@ -340,8 +343,8 @@ hipError_t hbm_copy_launch(const void* src, void* dst, size_t bytes, int blocks,
 hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
                             int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st);
 // one token's attention without the merge of its key partitions: their records (kAttnRec floats, [head][partition])
-// start kAttnCounterBytes into ws and their count goes to *parts (<= kAttnXMaxParts); with one partition out is
-// written instead and *parts is 1
+// start kAttnCounterBytes into ws and their count goes to *parts (<= kAttnXMaxParts); with one partition, and on a long
+// cache (merged there), out, which must be the kAttnCounterBytes-th byte of ws, is written instead and *parts is 1
 hipError_t attention_partials_launch(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int Hq,
                                      int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, int* parts,
                                      hipStream_t st);

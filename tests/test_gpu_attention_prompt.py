@@ -75,6 +75,37 @@ def test_prompt_attention_scales(cuda, scale):
     check(q, k, v, torch.arange(224, 320, device="cuda"), scale, 320)
 
 
+# few rows over long caches: the same kernel with up to 64 key partitions (64 rows a workgroup, or 32 beyond 128 rows), below
+# and above the lengths where it starts, positions well short of the cache's end, and partitions that hold no key
+@pytest.mark.parametrize("m,hq,hkv,L,last", [
+    (1, 28, 4, 4608, 4600), (1, 16, 2, 16384, 16383), (1, 12, 2, 10752, 40), (1, 4, 4, 32064, 32000), (2, 12, 2, 4096, 4095),
+    (3, 28, 4, 2048, 1029), (4, 16, 2, 2112, 2111), (16, 16, 2, 4096, 700), (17, 16, 2, 6400, 6399), (47, 16, 2, 2048, 2000),
+    (54, 28, 4, 2304, 2176)])
+def test_long_cache_attention(cuda, m, hq, hkv, L, last):
+    q, k, v = case(m, hq, hkv, L, m + last)
+    k[:, last + 1:] = float("nan")
+    v[:, last + 1:] = float("nan")
+    pos = torch.arange(last + 1 - m, last + 1, device="cuda")
+    one = check(q, k, v, pos, 128 ** -0.5, last + 1)
+    assert torch.equal(one, check(q, k, v, pos, 128 ** -0.5, last + 1))
+    check(q, k, v, torch.zeros(m, dtype=torch.long, device="cuda"), 128 ** -0.5, last + 1)
+
+
+def test_long_cache_attention_then_projection(cuda):
+    """lowbit_w4_attention_linear on a long cache: attention (merged by itself there), then the projection."""
+    from lowbit import _native
+    hq, hkv, L = 16, 2, 8192
+    q, k, v = case(1, hq, hkv, L, 4)
+    pos = torch.tensor([8000], device="cuda")
+    wq = ops.W4Weight.from_float(0.02 * torch.randn(512, hq * 128, device="cuda"), 128, ("mma",))
+    attn = torch.empty(1, hq * 128, dtype=torch.float16, device="cuda")
+    ext = ops.ext()
+    ext.attention(q, k, v, pos, attn, hq, hkv, L, 128 ** -0.5)
+    want = ext.w4_linear_fused(attn, wq.packed_mma, wq.scales, 128, _native.EPI_STORE)
+    got = ext.w4_attention_linear(q, k, v, pos, hq, hkv, L, 128 ** -0.5, wq.packed_mma, wq.scales, 128, _native.EPI_STORE)
+    assert torch.equal(got, want)
+
+
 def test_prompt_attention_of_growing_scores(cuda):
     """Every block of keys raises the rows' maximum far past the lag of the running reference, then lowers it again."""
     q, k, v = case(64, 16, 2, 1024, 9)
