@@ -90,9 +90,132 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
   if (lane == 0) scales[group] = best_sc;
 }
 
+// Groups of 32, 64 and 128 values: LPG = 4, 8 or 16 lanes a group, 8 consecutive values a lane, so that a wave quantizes
+// 16, 8 or 4 groups at once from 16-byte loads. The same bits as quantize_kernel: its lane l holds values 2 l and 2 l + 1,
+// so a lane here holds the pairs of one of its quads; their squared errors are added as wave_sum adds that quad, the rest
+// of its tree is the same tree over the lanes here, and its idle lanes add zeros.
+// The clip search evaluates v / scale for every value and candidate. A quotient is formed from the reciprocal y = RN(1 /
+// scale), one division per lane and candidate: q0 = RN(v y), r = v - q0 scale, q = RN(q0 + r y), Markstein's correction
+// (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).
+// It is the correctly rounded quotient: the scale is an fp16 value, so its 11 bits make r exact and keep v / scale at least
+// 2^-12 ulp away from every rounding boundary, far more than the ~2^-22 ulp that y's error can move the sum by; an infinite
+// scale, whose reciprocal says nothing, takes the division itself.
+// Bound: vector instructions (8 per value and candidate; the division took ~10 by itself). 11008 x 2048 fp16, 11
+// candidates, MI355X: quantize_kernel 208 us, 72 here.
+template <int kDtype>
+__device__ __forceinline__ void load8(const void* w, size_t i, float (&v)[8]) {
+  if constexpr (kDtype == 0) {
+    const f32x4 a = reinterpret_cast<const f32x4*>(w)[i / 4], b = reinterpret_cast<const f32x4*>(w)[i / 4 + 1];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = a[e], v[4 + e] = b[e];
+  } else {
+    const u32x4 t = load16(reinterpret_cast<const uint16_t*>(w) + i);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (kDtype == 1) {
+        v[2 * e] = (float)as_f16x2(t[e])[0];
+        v[2 * e + 1] = (float)as_f16x2(t[e])[1];
+      } else {
+        v[2 * e] = __builtin_bit_cast(float, t[e] << 16);
+        v[2 * e + 1] = __builtin_bit_cast(float, t[e] & 0xFFFF0000u);
+      }
+    }
+  }
+}
+
+template <int kDtype, int LPG>
+__global__ __launch_bounds__(256) void quantize_groups(const void* __restrict__ w, uint32_t* __restrict__ packed,
+                                                       f16* __restrict__ scales, long lanes, ClipGrid grid) {
+  const long gid = (long)blockIdx.x * 256 + threadIdx.x;
+  const bool live = gid < lanes;                            // a group's lanes are live together
+  float v[8];
+  load8<kDtype>(w, 8 * (size_t)(live ? gid : 0), v);
+  // over the lanes of a group: after the quad steps every quad is uniform, after lane ^ 7 every eight
+  auto over_group = [](float x, auto op) {
+    x = op(x, dpp<kQuadSwap1>(x));
+    x = op(x, dpp<kQuadSwap2>(x));
+    if (LPG >= 8) x = op(x, dpp<kRowHalfMirror>(x));
+    if (LPG >= 16) x = op(x, dpp<kRowMirror>(x));
+    return x;
+  };
+  float amax = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) amax = fmaxf(amax, fmaxf(fabsf(v[e]), fabsf(v[e + 1])));
+  amax = over_group(amax, [](float a, float b) { return fmaxf(a, b); });
+  auto quantize8 = [&](float scf, auto each) {              // each(e, quantized value), e = 0..7
+    if (__any(__builtin_isinf(scf))) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) each(e, quantize_one(v[e], scf));
+    } else {
+      const float y = 1.0f / scf;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float q0 = v[e] * y, r = fmaf(-q0, scf, v[e]);
+        each(e, fminf(fmaxf(__builtin_rintf(fmaf(r, y, q0)), -8.0f), 7.0f));
+      }
+    }
+  };
+  const int ncand = grid.n > 0 ? grid.n : 1;
+  f16 best_sc = (f16)1.0f;
+  float best_err = 0.f;
+  for (int ci = 0; ci < ncand; ++ci) {
+    const float a = grid.n > 0 ? grid.a[ci] : 1.0f;
+    const float num = a != 1.0f ? amax * a : amax;
+    f16 sc = (f16)(num / 7.0f);
+    if (sc == (f16)0.0f) sc = (f16)1.0f;
+    if (grid.n == 0) {
+      best_sc = sc;
+      break;
+    }
+    const float scf = (float)sc;
+    float d[8];
+    quantize8(scf, [&](int e, float q) { d[e] = q * scf - v[e]; });
+    float pair[4];                                          // as quantize_kernel's multiply and fused multiply-add round it
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float e1 = d[2 * e + 1];
+      pair[e] = fmaf(d[2 * e], d[2 * e], e1 * e1);
+      asm("" : "+v"(pair[e]));                              // (not fused into the sums below)
+    }
+    const float err = over_group((pair[0] + pair[1]) + (pair[2] + pair[3]), [](float x, float z) { return x + z; });
+    if (ci == 0 || err < best_err) {
+      best_err = err;
+      best_sc = sc;
+    }
+  }
+  if (!live) return;
+  const float scf = (float)best_sc;
+  uint32_t word = 0;
+  quantize8(scf, [&](int e, float q) { word |= (uint32_t)(int)(q + 8.0f) << (4 * e); });
+  packed[gid] = word;
+  if (gid % LPG == 0) scales[gid / LPG] = best_sc;
+}
+
+namespace {
+template <int kDtype>
+hipError_t launch_groups(const void* w, uint8_t* packed, f16* scales, long lanes, int G, const ClipGrid& grid,
+                         hipStream_t st) {
+  const dim3 gr((unsigned)((lanes + 255) / 256)), block(256);
+  uint32_t* words = reinterpret_cast<uint32_t*>(packed);
+  if (G == 32) return launch(quantize_groups<kDtype, 4>, gr, block, 0, st, w, words, scales, lanes, grid);
+  if (G == 64) return launch(quantize_groups<kDtype, 8>, gr, block, 0, st, w, words, scales, lanes, grid);
+  return launch(quantize_groups<kDtype, 16>, gr, block, 0, st, w, words, scales, lanes, grid);
+}
+}  // namespace
+
 hipError_t quantize_launch(const void* w, int dtype, uint8_t* packed, f16* scales, int N, int K, int G,
                            const ClipGrid& grid, hipStream_t st) {
   const size_t groups = (size_t)N * (K / G);
+  // other group sizes, and tensors that 16-byte loads or 4-byte stores do not fit, take the kernel of a wave per group
+  if ((G == 32 || G == 64 || G == 128) && (reinterpret_cast<uintptr_t>(w) & 15) == 0 &&
+      (reinterpret_cast<uintptr_t>(packed) & 3) == 0) {
+    const long lanes = (long)groups * (G / 8);
+    switch (dtype) {
+      case 0: return launch_groups<0>(w, packed, scales, lanes, G, grid, st);
+      case 1: return launch_groups<1>(w, packed, scales, lanes, G, grid, st);
+      default: return launch_groups<2>(w, packed, scales, lanes, G, grid, st);
+    }
+  }
   dim3 gr((unsigned)((groups + 3) / 4)), block(256);
   switch (dtype) {
     case 0: return launch(quantize_kernel<0>, gr, block, 0, st, w, packed, scales, N, K, G, grid);
