@@ -21,6 +21,7 @@ DTYPE_F32, DTYPE_F16, DTYPE_BF16 = 0, 1, 2
 
 _LIB = None
 _FORMAT_LIB = None
+torch = None                            # imported with the kernels (NativeExt): the format functions need no torch
 
 _i64, _int, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_void_p
 SIGNATURES = {
@@ -191,18 +192,18 @@ def workspace(device, stream, nbytes=WORKSPACE_BYTES, tag=""):
 def _check_epilogue(epilogue, aux, m, n, device):
     """aux must match what the kernels read: bias [N] or residual [M, N], fp16, contiguous, on x's GPU (the C ABI
     cannot check its size)."""
-    import torch
-    if epilogue not in (EPI_STORE, EPI_BIAS, EPI_RESIDUAL, EPI_SILU_MUL):
+    if epilogue == EPI_STORE or epilogue == EPI_SILU_MUL:
+        return
+    if epilogue not in (EPI_BIAS, EPI_RESIDUAL):
         raise RuntimeError("unknown epilogue")
-    if epilogue in (EPI_BIAS, EPI_RESIDUAL):
-        if aux is None:
-            raise RuntimeError("the bias and residual epilogues need aux")
-        if aux.dtype != torch.float16 or not aux.is_contiguous() or aux.device != device:
-            raise RuntimeError("aux must be a contiguous float16 tensor on the same GPU")
-        if epilogue == EPI_BIAS and aux.numel() != n:
-            raise RuntimeError(f"bias must hold N={n} values, got {aux.numel()}")
-        if epilogue == EPI_RESIDUAL and (aux.dim() != 2 or tuple(aux.shape) != (m, n)):
-            raise RuntimeError(f"the residual must be [M, N] = [{m}, {n}], got {list(aux.shape)}")
+    if aux is None:
+        raise RuntimeError("the bias and residual epilogues need aux")
+    if aux.dtype is not torch.float16 or not aux.is_contiguous() or aux.device != device:
+        raise RuntimeError("aux must be a contiguous float16 tensor on the same GPU")
+    if epilogue == EPI_BIAS and aux.numel() != n:
+        raise RuntimeError(f"bias must hold N={n} values, got {aux.numel()}")
+    if epilogue == EPI_RESIDUAL and (aux.dim() != 2 or tuple(aux.shape) != (m, n)):
+        raise RuntimeError(f"the residual must be [M, N] = [{m}, {n}], got {list(aux.shape)}")
 
 
 def _need(t, name, dtype, shape, device):
@@ -223,53 +224,72 @@ def _check_norm(norm, k, device):
 
 
 def _check_tensors(x, w, s, group):
-    """The tensor-metadata half of the reference's check() (csrc/w4_gemv.cu:312-325); sizes are checked natively."""
-    import torch
+    """The tensor-metadata half of the reference's check() (csrc/w4_gemv.cu:312-325); sizes are checked natively.
+    Returns (M, N, K, GPU index). Every projection called from Python pays for this, so it reads each property once and
+    compares GPU indices rather than device objects."""
     if not (x.is_cuda and w.is_cuda and s.is_cuda):
         raise RuntimeError("tensors must be on the GPU")
-    if w.device != x.device or s.device != x.device:
+    index = x.get_device()
+    if w.get_device() != index or s.get_device() != index:
         raise RuntimeError("x, w and scales must be on the same GPU")
     if group <= 0:
         raise RuntimeError("group size must be positive")
-    if x.dtype != torch.float16 or s.dtype != torch.float16 or w.dtype != torch.uint8:
+    if x.dtype is not torch.float16 or s.dtype is not torch.float16 or w.dtype is not torch.uint8:
         raise RuntimeError("x and scales must be float16, packed weights uint8")
     if not (x.is_contiguous() and w.is_contiguous() and s.is_contiguous()):
         raise RuntimeError("tensors must be contiguous")
-    if x.dim() != 2 or w.dim() != 2 or s.dim() != 2:
+    xs, wsh, ss = x.shape, w.shape, s.shape
+    if len(xs) != 2 or len(wsh) != 2 or len(ss) != 2:
         raise RuntimeError("x [M,K], w [N,K/2], scales [N,K/G]")
-    k = x.shape[1]
+    m, k = xs
+    n = wsh[0]
     if group % 32 or k % group:
         raise RuntimeError("K must be a multiple of the group size, itself a multiple of 32")
-    if w.shape[1] * 2 != k or s.shape[0] != w.shape[0] or s.shape[1] != k // group:
+    if wsh[1] * 2 != k or ss[0] != n or ss[1] != k // group:
         raise RuntimeError("shape mismatch")
+    return m, n, k, index
+
+
+def _launch(index, call, nbytes=0):
+    """call(stream, workspace address, workspace bytes) on GPU `index`, made current for the call, with that GPU's current
+    stream and its workspace of `nbytes` (0: none); raises on a non-zero status. The launch path of the projections: the
+    current device and stream come from torch's plain getters, as integers."""
+    if torch._C._cuda_getDevice() != index:
+        with torch.cuda.device(index):
+            return _launch(index, call, nbytes)
+    stream = torch._C._cuda_getCurrentRawStream(index)
+    if nbytes:
+        ws = _WORKSPACES.get((index, stream or None, nbytes, ""))   # workspace()'s key
+        if ws is None:
+            ws = workspace(torch.device("cuda", index), ctypes.c_void_p(stream), nbytes)
+        rc = call(stream, ws.data_ptr(), nbytes)
+    else:
+        rc = call(stream, None, 0)
+    if rc:
+        check(rc)
 
 
 class NativeExt:
     """The reference's extension surface (w4_gemv / w4_gemm_tc / w4_dequant) on the gfx950 library."""
 
     def __init__(self):
+        global torch
+        import torch
         self.lib = lib()
 
     def w4_gemv(self, x, w, s, group, version, rows_per_warp=0):
-        import torch
-        _check_tensors(x, w, s, group)
-        m, n = x.shape[0], w.shape[0]
-        y = torch.empty((m, n), dtype=torch.float16, device=x.device)
-        with _DeviceGuard(x.device):
-            check(self.lib.lowbit_w4_gemv(ptr(x), ptr(w), ptr(s), ptr(y), m, n, x.shape[1], group, int(version),
-                                          int(rows_per_warp), _stream(x.device)))
+        m, n, k, index = _check_tensors(x, w, s, group)
+        y = x.new_empty((m, n))
+        _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemv(
+            x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(version), int(rows_per_warp), stream))
         return y
 
     def w4_gemm_tc(self, x, w, s, group, row_tiles=0):
-        import torch
-        _check_tensors(x, w, s, group)
-        m, n = x.shape[0], w.shape[0]
-        y = torch.empty((m, n), dtype=torch.float16, device=x.device)
-        with _DeviceGuard(x.device):
-            st = _stream(x.device)
-            ws = workspace(x.device, st)
-            check(self.lib.lowbit_w4_gemm_mfma(ptr(x), ptr(w), ptr(s), ptr(y), m, n, x.shape[1], group, int(row_tiles),
-                                               ptr(ws), ws.numel(), st))
+        m, n, k, index = _check_tensors(x, w, s, group)
+        y = x.new_empty((m, n))
+        _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemm_mfma(
+            x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(row_tiles), ws, nbytes, stream),
+            WORKSPACE_BYTES)
         return y
 
     def w4_gemm_tc_noalloc(self, x, w, s, group, row_tiles=0):
@@ -343,42 +363,34 @@ class NativeExt:
         ([M, N], or [M, N / 2] for EPI_SILU_MUL). `out` may be given (for EPI_RESIDUAL it may be `aux` itself).
         norm = (weight, eps): project RMSNorm(x) * weight instead of x, normalized in the kernel (K <= 16384 for one
         row; K <= 8192 for 2..64 rows, with lowbit_rmsnorm's bits)."""
-        import torch
-        _check_tensors(x, w, s, group)
-        m, n = x.shape[0], w.shape[0]
-        cols = n // 2 if epilogue == EPI_SILU_MUL else n
-        y = out if out is not None else torch.empty((m, cols), dtype=torch.float16, device=x.device)
-        if y.shape != (m, cols) or y.dtype != torch.float16 or not y.is_contiguous() or y.device != x.device:
-            raise RuntimeError("out must be a contiguous float16 [M, N] (or [M, N/2] for silu-mul) tensor")
+        m, n, k, index = _check_tensors(x, w, s, group)
+        y = self._output(x, m, n, epilogue, out)
         _check_epilogue(epilogue, aux, m, n, x.device)
-        _check_norm(norm, x.shape[1], x.device)
-        with _DeviceGuard(x.device):
-            st = _stream(x.device)
-            ws = workspace(x.device, st)
-            nw, eps = norm if norm is not None else (None, 0.0)
-            check(self.lib.lowbit_w4_linear_fused(ptr(x), ptr(w), ptr(s), ptr(y), m, n, x.shape[1], group,
-                                                  int(epilogue), ptr(aux) if aux is not None else None,
-                                                  ptr(nw) if nw is not None else None, float(eps), ptr(ws),
-                                                  ws.numel(), st))
+        _check_norm(norm, k, x.device)
+        nw, eps = norm if norm is not None else (None, 0.0)
+        _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_linear_fused(
+            x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(epilogue),
+            aux.data_ptr() if aux is not None else None, nw.data_ptr() if nw is not None else None, float(eps), ws, nbytes,
+            stream), WORKSPACE_BYTES)
         return y
+
+    def _output(self, x, m, n, epilogue, out):
+        cols = n // 2 if epilogue == EPI_SILU_MUL else n
+        if out is None:
+            return x.new_empty((m, cols))
+        if out.shape != (m, cols) or out.dtype != torch.float16 or not out.is_contiguous() or out.device != x.device:
+            raise RuntimeError("out must be a contiguous float16 [M, N] (or [M, N/2] for silu-mul) tensor")
+        return out
 
     def w4_gemm_prefill(self, x, w, s, group, epilogue=EPI_STORE, aux=None, out=None):
         """x [M, K] (any M, meant for M > 64) times the MFMA-layout weight, int4 read directly, with the epilogue
         fused into the store; returns y ([M, N], or [M, N / 2] for EPI_SILU_MUL)."""
-        import torch
-        _check_tensors(x, w, s, group)
-        m, n = x.shape[0], w.shape[0]
-        cols = n // 2 if epilogue == EPI_SILU_MUL else n
-        y = out if out is not None else torch.empty((m, cols), dtype=torch.float16, device=x.device)
-        if y.shape != (m, cols) or y.dtype != torch.float16 or not y.is_contiguous() or y.device != x.device:
-            raise RuntimeError("out must be a contiguous float16 [M, N] (or [M, N/2] for silu-mul) tensor")
+        m, n, k, index = _check_tensors(x, w, s, group)
+        y = self._output(x, m, n, epilogue, out)
         _check_epilogue(epilogue, aux, m, n, x.device)
-        with _DeviceGuard(x.device):
-            st = _stream(x.device)
-            ws = workspace(x.device, st, PREFILL_WORKSPACE_BYTES)
-            check(self.lib.lowbit_w4_gemm_prefill(ptr(x), ptr(w), ptr(s), ptr(y), m, n, x.shape[1], group,
-                                                  int(epilogue), ptr(aux) if aux is not None else None, ptr(ws),
-                                                  ws.numel(), st))
+        _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemm_prefill(
+            x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(epilogue),
+            aux.data_ptr() if aux is not None else None, ws, nbytes, stream), PREFILL_WORKSPACE_BYTES)
         return y
 
     def rmsnorm(self, x, weight, eps, out=None):

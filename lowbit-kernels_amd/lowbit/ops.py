@@ -235,7 +235,8 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     if bias is not None:                      # one bias for every route: fp16 [N] on x's device
         if bias.numel() != wq.n:
             raise ValueError(f"bias must hold N={wq.n} values, got shape {list(bias.shape)}")
-        bias = bias.reshape(wq.n).to(device=x.device, dtype=torch.float16).contiguous()
+        if bias.dim() != 1 or bias.dtype is not torch.float16 or bias.device != x.device or not bias.is_contiguous():
+            bias = bias.reshape(wq.n).to(device=x.device, dtype=torch.float16).contiguous()
     if version == 0:
         v = auto_version(m, wq)
     elif version in MAX_ROWS:
