@@ -852,79 +852,81 @@ __global__ __launch_bounds__(kPickThreads) void head_pick_kernel(const uint64_t*
 constexpr int kHeadRows = 2;                                // RW: rows per wave (4 waves a workgroup)
 
 // fp16-weight MFMA GEMV for the head beyond 8 rows (up to 64: MT 16-row activation tiles), where the dot2 kernel above
-// turns ALU-bound. Each wave owns one 16-row tile of W, the MFMA's A, straight from global: lane (r, q) takes row r,
-// k = 128 c + 32 s + 8 q + 0..7 as k-step s of chunk c, so one load instruction reads 64 contiguous bytes of each of
-// 16 rows (kF16wSlots chunks in flight, default cache policy: with non-temporal loads the half-used 128-byte lines
-// were fetched twice, 199 against 135 us). The workgroup's four waves share each 128-k chunk of x (B, the same k
-// order), staged by all 256 threads into one of two LDS buffers (16-byte pieces XOR-swizzled by row, so a B
-// fragment's 16 rows hit different banks) while the previous chunk is consumed, one barrier per chunk; rows past M
-// read zeros and are not stored. Lane l holds y[16 mt + l % 16][16 t + 4 (l / 16) + v], v = 0..3. On the 151936 x 2048
-// head (3 cold copies): 16 rows 135 us against 204 for hipBLASLt, 32 rows 142 against 146, 48 rows 152 against 144
-// (hipBLASLt keeps those), the same as with x staged whole in LDS at 16 rows.
-constexpr int kF16wSlots = 4;
+// turns ALU-bound. Each wave owns one 16-row tile of W, the MFMA's A; the workgroup's four waves share x, the B. Both
+// stream through LDS in 128-k chunks by direct-to-LDS loads, D chunks deep: a wave-load takes 256 contiguous
+// bytes of each of 4 rows, non-temporal for W, where the fragments read from memory directly (lane (r, q) its own row) took
+// 64 bytes of 16 rows, half of each 128-byte line. A row's sixteen 16-byte blocks are permuted by the row (block b at
+// b ^ f16w_swz(row % 16)), so a fragment's rows meet different banks; lane (r, q) takes block 4 q + s as k-step s. One
+// barrier a chunk: it makes the next chunk's x visible and frees the slot consumed before; loads complete in issue order,
+// so waiting for all but the newest D - 2 chunks' loads means that the chunk has landed. Rows past N and M read
+// zeros. Lane l holds y[16 mt + l % 16][16 t + 4 (l / 16) + v], v = 0..3.
+// Bound: HBM. 151936 x 2048 head (622 MB, 3 cold copies), MI355X, us (direct fragments -> this; hipBLASLt): 16 rows
+// 134 -> 104 (205), 32 rows 145 -> 114 (147), 48 rows 156 -> 133 (144), 64 rows 166 -> 144 (154); one more slot at 16
+// rows, which costs the second workgroup per CU, 110.
+constexpr int f16w_slots(int MT) { return MT == 1 ? 4 : 3; }   // (80 KB of LDS: two workgroups per CU)
+constexpr int f16w_swz(int r) { return ((r & 3) << 2) | (r >> 2); }
 template <int MT>
 __global__ __launch_bounds__(256) void gemm_f16w_rows_kernel(const f16* __restrict__ x, const f16* __restrict__ w,
                                                              f16* __restrict__ y, int M, int N, int K) {
-  constexpr int kRows = 16 * MT, kBuf = kRows * 256;        // one staged chunk of x: kRows rows x 256 bytes
-  constexpr int XP = kRows * 16 / 256;                     // 16-byte pieces a thread stages per chunk
+  constexpr int D = f16w_slots(MT), kTile = 16 * 256;           // bytes of 16 rows of a chunk
+  constexpr int kSlot = (4 + MT) * kTile;                   // a chunk: the waves' W tiles, then x
+  constexpr int kLoads = 4 + MT;                            // a wave's loads of a chunk
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4, KC = K >> 7;
   const int n0 = 16 * (blockIdx.x * 4 + wave);
   const int rows = max(0, min(16, N - n0));
-  const __amdgpu_buffer_rsrc_t wr = make_rsrc(w + (size_t)min(n0, N) * K, (uint32_t)(rows * K * 2));
+  // (hipcc multiplies 64-bit sizes in vector registers; the resource of a direct-to-LDS load must be scalar)
+  const uint64_t first = (uint64_t)min(n0, N) * (uint64_t)K;
+  const uint64_t first_s = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(first >> 32)) << 32) |
+                           (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)first);
+  const __amdgpu_buffer_rsrc_t wr = make_rsrc(w + first_s, (uint32_t)__builtin_amdgcn_readfirstlane(rows * K * 2));
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(x, (uint32_t)(M * K * 2));
-  const int woff = r < rows ? 2 * (r * K + 8 * q) : kOutOfRange;
-  auto slot = [](int row, int piece) { return 16 * (16 * row + (piece ^ (row & 15))); };   // byte offset in a buffer
-  int xoff[XP], xsl[XP];
+  // W load u of a wave: rows 4 u + lane / 16, slot lane % 16 of the row. x load mt: row 16 mt + tid / 16, slot tid % 16
+  int woff[4], xoff[MT];
 #pragma unroll
-  for (int u = 0; u < XP; ++u) {                            // piece p = tid + 256 u: row p / 16, piece p % 16
-    const int p = tid + 256 * u;
-    xoff[u] = (p >> 4) < M ? 2 * ((p >> 4) * K + 8 * (p & 15)) : kOutOfRange;
-    xsl[u] = slot(p >> 4, p & 15);
+  for (int u = 0; u < 4; ++u) woff[u] = 2 * ((4 * u + q) * K + 8 * (r ^ f16w_swz(4 * u + q)));
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt) {
+    const int row = 16 * mt + (tid >> 4);
+    xoff[mt] = row < M ? 2 * (row * K + 8 * ((tid & 15) ^ f16w_swz(tid >> 4))) : kOutOfRange - 256 * KC;
   }
-  u32x4 ring[kF16wSlots][4], rx[XP];
-  auto issue = [&](int d, int c) {
+  const uint32_t base = lds_addr(smem);
+  auto issue = [&](int d, int c) {                          // kLoads loads, always (chunks past the end read zeros)
+    const bool live = c < KC;
+    const uint32_t at = base + d * kSlot;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) ring[d][s] = buffer_load16(wr, c < KC ? woff + 2 * (128 * c + 32 * s) : kOutOfRange);
+    for (int u = 0; u < 4; ++u) dma16_nt(wr, live ? woff[u] + 256 * c : kOutOfRange, at + wave * kTile + 1024 * u);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) dma16(xr, live ? xoff[mt] + 256 * c : kOutOfRange, at + (4 + mt) * kTile + 1024 * wave);
   };
-  auto load_x = [&](int c) {
 #pragma unroll
-    for (int u = 0; u < XP; ++u) rx[u] = buffer_load16(xr, c < KC ? xoff[u] + 256 * c : kOutOfRange);
-  };
-  auto stage_x = [&](int b) {
-#pragma unroll
-    for (int u = 0; u < XP; ++u) *reinterpret_cast<u32x4*>(smem + b * kBuf + xsl[u]) = rx[u];
-  };
-  load_x(0);
-#pragma unroll
-  for (int d = 0; d < kF16wSlots; ++d) issue(d, d);
-  stage_x(0);
-  __syncthreads();
+  for (int d = 0; d < D - 1; ++d) issue(d, d);
   f32x4 acc[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < KC; c0 += kF16wSlots) {
+  for (int c0 = 0; c0 < KC; c0 += D) {
 #pragma unroll
-    for (int d = 0; d < kF16wSlots; ++d) {
+    for (int d = 0; d < D; ++d) {
       const int c = c0 + d;
       if (c < KC) {                                         // uniform: every wave runs the same chunks
-        load_x(c + 1);
-        const uint8_t* xb = smem + (c & 1) * kBuf;
+        lds_wait_barrier<(D - 2) * kLoads>();               // chunk c has landed in every wave; slot c - 1 is free
+        issue((d + D - 1) % D, c + D - 1);
+        const uint8_t* slot = smem + d * kSlot;
 #pragma unroll
-        for (int s = 0; s < 4; ++s)
+        for (int s = 0; s < 4; ++s) {
+          const int at = 256 * r + 16 * ((4 * q + s) ^ f16w_swz(r));
+          const f16x8 a = *reinterpret_cast<const f16x8*>(slot + wave * kTile + at);
 #pragma unroll
           for (int mt = 0; mt < MT; ++mt) {
-            const u32x4 b = *reinterpret_cast<const u32x4*>(xb + slot(16 * mt + r, 4 * s + q));
-            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, ring[d][s]),
-                                                             __builtin_bit_cast(f16x8, b), acc[mt], 0, 0, 0);
+            const f16x8 b = *reinterpret_cast<const f16x8*>(slot + (4 + mt) * kTile + at);
+            acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[mt], 0, 0, 0);
           }
-        issue(d, c + kF16wSlots);
-        if (c + 1 < KC) stage_x((c + 1) & 1);
-        __syncthreads();
+        }
       }
     }
   }
+  vm_drain();                                               // no load into LDS is left in flight
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) {
     const int m = 16 * mt + r, n = n0 + 4 * q;
@@ -942,15 +944,20 @@ __global__ __launch_bounds__(256) void gemm_f16w_rows_kernel(const f16* __restri
   }
 }
 
+template <int MT>
+hipError_t launch_f16w_rows(const f16* x, const f16* w, f16* y, int M, int N, int K, hipStream_t st) {
+  constexpr size_t lds = (size_t)f16w_slots(MT) * (4 + MT) * 16 * 256;
+  static const hipError_t attr = allow_lds(gemm_f16w_rows_kernel<MT>, lds);
+  if (attr != hipSuccess) return attr;
+  return launch(gemm_f16w_rows_kernel<MT>, dim3((unsigned)((N + 63) / 64)), dim3(256), lds, st, x, w, y, M, N, K);
+}
+
 hipError_t gemm_f16w_rows_launch(const f16* x, const f16* w, f16* y, int M, int N, int K, hipStream_t st) {
-  const dim3 grid((unsigned)((N + 63) / 64)), block(256);
-  const int MT = (M + 15) / 16;
-  const size_t lds = (size_t)2 * 16 * MT * 256;
-  switch (MT) {
-    case 1: return launch(gemm_f16w_rows_kernel<1>, grid, block, lds, st, x, w, y, M, N, K);
-    case 2: return launch(gemm_f16w_rows_kernel<2>, grid, block, lds, st, x, w, y, M, N, K);
-    case 3: return launch(gemm_f16w_rows_kernel<3>, grid, block, lds, st, x, w, y, M, N, K);
-    default: return launch(gemm_f16w_rows_kernel<4>, grid, block, lds, st, x, w, y, M, N, K);
+  switch ((M + 15) / 16) {
+    case 1: return launch_f16w_rows<1>(x, w, y, M, N, K, st);
+    case 2: return launch_f16w_rows<2>(x, w, y, M, N, K, st);
+    case 3: return launch_f16w_rows<3>(x, w, y, M, N, K, st);
+    default: return launch_f16w_rows<4>(x, w, y, M, N, K, st);
   }
 }
 
@@ -969,8 +976,8 @@ hipError_t gemv_f16_launch(const f16* x, const f16* w, f16* y, int M, int N, int
     case 3: return launch_head<3, kHeadRows, kHeadChunks>(x, w, y, 3, N, K, st);
     case 4: return launch_head<4, kHeadRows, kHeadChunks>(x, w, y, 4, N, K, st);
     // more rows: 8 weight rows per wave, two chunks in flight (the head, 3 cold copies: 8 rows 119.5 us against
-    // 126.6 for 4 per wave and 163.7 for 2; hipBLASLt 203.6. 16 rows: 206 us, level with hipBLASLt's 204: the dot2
-    // sequence per weight byte grows with the rows and the kernel turns ALU-bound)
+    // 126.6 for 4 per wave and 163.7 for 2; hipBLASLt 203.6). The MFMA kernel would take 101 there, but up to 8 rows a
+    // row has the bits it has alone
     default: {
       const bool x_fits = (size_t)M * K * 2 <= 65536;      // the dot2 kernels stage x whole
       if (M <= 8 && x_fits) return launch_head<8, 8, 2>(x, w, y, M, N, K, st);

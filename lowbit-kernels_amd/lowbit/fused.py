@@ -188,9 +188,9 @@ class FusedQwen2:
         return self.hidden * 2 <= 65536
 
     def logits(self, xn, pick=None):
-        """The tied fp16 head: the library's fp16 GEMV for up to 32 rows (hipBLASLt streams the head at ~3 TB/s at
-        these shapes: 94 against 202 us at one row, 120 against 204 at 8, 135 against 204 at 16, 142 against 146 at
-        32), hipBLASLt beyond (144 against 152 at 48). pick = (tokens, positions[, out_tokens, out_count, h_next]),
+        """The tied fp16 head: the library's fp16 GEMV for up to 32 rows, or 64 while hidden <= 2048 (against hipBLASLt,
+        3B head: 94 and 203 us at one row, 119 and 204 at 8, 104 and 205 at 16, 114 and 147 at 32, 144 and 154 at 64;
+        7B: 165 and 230 at 16, 181 and 248 at 32), hipBLASLt beyond (7B at 48 rows 212 and 200). pick = (tokens, positions[, out_tokens, out_count, h_next]),
         one row (head_picks()): the GEMV also writes the greedy pick to tokens[0], advances positions[0] and, given
         the rest, appends the pick to out_tokens and writes its embedding row to h_next (the next step's input)."""
         if pick is not None:
@@ -199,7 +199,7 @@ class FusedQwen2:
                 more = dict(out_tokens=pick[2], out_count=pick[3], embed=self.embed, h_out=pick[4])
             return ops.ext().f16_gemv_pick(xn, self.head, pick[0], pick[1], **more)
         m, k = xn.shape
-        if (m <= 8 and m * k * 2 <= 65536) or (m <= 32 and k % 128 == 0):
+        if (m <= 8 and m * k * 2 <= 65536) or (m <= (64 if k <= 2048 else 32) and k % 128 == 0):
             return ops.ext().f16_gemv(xn, self.head)
         return F.linear(xn, self.head)
 
