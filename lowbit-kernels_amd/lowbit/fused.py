@@ -210,7 +210,8 @@ class FusedQwen2:
         [M, hidden] when the caller already holds them (it becomes the residual stream, overwritten)."""
         ext = ops.ext()
         m = tokens.shape[0]
-        h = F.embedding(tokens, self.embed) if h is None else h
+        if h is None:                                         # (up to 16 tokens F.embedding picks a small-index kernel, 12
+            h = torch.gather(self.embed, 0, tokens[:, None].expand(m, self.hidden))   # us at 16 against 5; same checks)
         xn = torch.empty_like(h)
         q = torch.empty(m, self.hq, self.head_dim, dtype=torch.float16, device=h.device)
         attn = torch.empty(m, self.hq * self.head_dim, dtype=torch.float16, device=h.device)
@@ -352,7 +353,7 @@ class FusedDecoder:
         if self.pos + self.chunk > self.f.max_len:
             raise ValueError("the cache is full")
         self.tokens.copy_(tokens.view(self.chunk))
-        self.positions.copy_(self.offsets + self.pos)
+        torch.add(self.offsets, self.pos, out=self.positions)
         if self.h is not None:
             torch.index_select(self.f.embed, 0, self.tokens, out=self.h)
         self.graph.replay()
