@@ -204,21 +204,35 @@ def prefill(x, wq):
     return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group)
 
 
+def _prefill_without_blas(m, wq):
+    """The part of prefill_path that holds whatever is asked of x: the rest keeps dequantize + BLAS for calls that
+    torch differentiates or transforms (_plain)."""
+    return (wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS
+            or (m <= AUTO_PREFILL_NARROW_ROWS and wq.n <= AUTO_PREFILL_NARROW and wq.k <= AUTO_PREFILL_NARROW))
+
+
 def prefill_path(m, wq):
     """True when linear() sends m rows to the int4 prefill GEMM rather than dequantize + BLAS (auto routing only)."""
     if auto_version(m, wq) is not None or wq.packed_mma is None:
         return False
-    if wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS:
+    if _prefill_without_blas(m, wq):
         return True
     if m > AUTO_PREFILL_NARROW_ROWS:
         return False
-    narrow = wq.n <= AUTO_PREFILL_NARROW
-    if narrow and wq.k <= AUTO_PREFILL_NARROW:
-        return True
-    if m <= AUTO_PREFILL_WIDE_ROWS and (narrow or wq.n > AUTO_PREFILL_WIDE_N):
+    if m <= AUTO_PREFILL_WIDE_ROWS and (wq.n <= AUTO_PREFILL_NARROW or wq.n > AUTO_PREFILL_WIDE_N):
         return True
     tiles = -(-m // 256) * -(-wq.n // 256)
     return tiles > 256 and tiles < AUTO_PREFILL_FILL * 256 * -(-tiles // 256)
+
+
+def _plain(x):
+    """True when x is an fp16 matrix of which only the values matter: no gradient, autocast, forward-mode level, function
+    transform, trace, tensor subclass or third dimension that the BLAS GEMM, a torch operator, would serve and a kernel
+    call would not."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and x.dim() == 2 and x.dtype is torch.float16
+            and not (x.requires_grad and torch.is_grad_enabled()) and not torch.is_autocast_enabled()
+            and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x))
 
 
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
@@ -249,7 +263,7 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
         return ext().w4_linear_fused(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias)
     if v is not None:
         y = gemv(x, wq, v)
-    elif version == 0 and prefill_path(m, wq):
+    elif version == 0 and prefill_path(m, wq) and (_prefill_without_blas(m, wq) or _plain(x)):
         if bias is not None:
             return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias)
         y = prefill(x, wq)

@@ -1,0 +1,68 @@
+"""linear()'s route above AUTO_PREFILL_ROWS rows (CPU: the kernels are replaced by a recorder and a plain product): plain
+calls take the int4 prefill GEMM where prefill_path says, calls that torch differentiates or transforms keep dequantize +
+BLAS there and so their gradients, tangents and batches."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.autograd.forward_ad as fwad
+
+from lowbit import ops
+
+N, K, M = 8320, 128, 600                                    # a wide layer, more rows than AUTO_PREFILL_ROWS
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    w = torch.randn(N, K, generator=torch.Generator().manual_seed(1)).half()
+    taken = []
+
+    def fake(name, result):
+        def call(*args, **kwargs):
+            taken.append(name)
+            return result(*args)
+        return call
+    monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq: x.detach() @ w.t()))
+    monkeypatch.setattr(ops, "dequant", fake("dequant", lambda *a: w))
+    wq = SimpleNamespace(n=N, k=K, packed=None, packed_v3=None, packed_mma=object())
+    assert ops.prefill_path(M, wq) and not ops._prefill_without_blas(M, wq)
+    return wq, w, taken
+
+
+def test_plain_calls_take_the_int4_gemm(layer):
+    wq, w, taken = layer
+    x = torch.randn(M, K).half()
+    ops.linear(x, wq)
+    with torch.no_grad():
+        ops.linear(x.clone().requires_grad_(), wq)
+    ops.linear(torch.nn.Parameter(x, requires_grad=False), wq)
+    assert taken == ["prefill"] * 3
+
+
+def near(a, b):                                             # fp16 products of 128 unit-variance terms
+    return torch.allclose(a.float(), b.float(), rtol=2e-2, atol=0.1)
+
+
+def test_transformed_calls_keep_blas(layer):
+    wq, w, taken = layer
+    x = torch.randn(M, K).half().requires_grad_()
+    ops.linear(x, wq).backward(torch.eye(M, N).half())
+    assert near(x.grad, w[:M])
+    with fwad.dual_level():
+        t = torch.randn(M, K).half()
+        out = ops.linear(fwad.make_dual(torch.randn(M, K).half(), t), wq)
+        assert near(fwad.unpack_dual(out).tangent, t @ w.t())
+    xs = torch.randn(2, M, K).half()
+    assert near(torch.func.vmap(lambda a: ops.linear(a, wq))(xs), xs @ w.t())
+    x3 = torch.randn(M, 2, K).half()
+    assert near(ops.linear(x3, wq), x3 @ w.t())
+    assert taken == ["dequant"] * 4
+
+
+@pytest.mark.parametrize("m,n,k,want", [
+    (512, 8192, 2048, True), (513, 8192, 2048, False), (513, 4096, 8960, True), (1024, 8193, 2048, True),
+    (1025, 4096, 8960, False), (1024, 4097, 2048, False), (1400, 22016, 2048, True), (1400, 18944, 3584, False),
+    (2048, 18944, 3584, True), (2048, 22016, 2048, False), (2048, 16384, 3584, False), (2049, 18944, 3584, False),
+    (2048, 4096, 4096, True), (2049, 4096, 4096, False), (5000, 256, 16384, True)])
+def test_rule(m, n, k, want):
+    assert ops.prefill_path(m, SimpleNamespace(n=n, k=k, packed=None, packed_v3=None, packed_mma=object())) is want
