@@ -250,6 +250,14 @@ def _check_tensors(x, w, s, group):
     return m, n, k, index
 
 
+def _output_rows(x, m, n):
+    """An uninitialised fp16 [m, n] tensor on x's GPU: a plain Tensor also where x is of a subclass, whose new_empty would
+    answer with its own type (new_empty is the cheaper call, so plain inputs take it)."""
+    if type(x) is torch.Tensor:
+        return x.new_empty((m, n))
+    return torch.empty((m, n), dtype=torch.float16, device=x.device)
+
+
 def _launch(index, call, nbytes=0):
     """call(stream, workspace address, workspace bytes) on GPU `index`, made current for the call, with that GPU's current
     stream and its workspace of `nbytes` (0: none); raises on a non-zero status. The launch path of the projections: the
@@ -279,14 +287,14 @@ class NativeExt:
 
     def w4_gemv(self, x, w, s, group, version, rows_per_warp=0):
         m, n, k, index = _check_tensors(x, w, s, group)
-        y = x.new_empty((m, n))
+        y = _output_rows(x, m, n)
         _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemv(
             x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(version), int(rows_per_warp), stream))
         return y
 
     def w4_gemm_tc(self, x, w, s, group, row_tiles=0):
         m, n, k, index = _check_tensors(x, w, s, group)
-        y = x.new_empty((m, n))
+        y = _output_rows(x, m, n)
         _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemm_mfma(
             x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(row_tiles), ws, nbytes, stream),
             WORKSPACE_BYTES)
@@ -377,7 +385,7 @@ class NativeExt:
     def _output(self, x, m, n, epilogue, out):
         cols = n // 2 if epilogue == EPI_SILU_MUL else n
         if out is None:
-            return x.new_empty((m, cols))
+            return _output_rows(x, m, cols)
         if out.shape != (m, cols) or out.dtype != torch.float16 or not out.is_contiguous() or out.device != x.device:
             raise RuntimeError("out must be a contiguous float16 [M, N] (or [M, N/2] for silu-mul) tensor")
         return out

@@ -7,7 +7,7 @@ import pytest
 import torch
 import torch.autograd.forward_ad as fwad
 
-from lowbit import ops
+from lowbit import _native, ops
 
 N, K, M = 8320, 128, 600                                    # a wide layer, more rows than AUTO_PREFILL_ROWS
 
@@ -66,3 +66,13 @@ def test_transformed_calls_keep_blas(layer):
     (2048, 4096, 4096, True), (2049, 4096, 4096, False), (5000, 256, 16384, True)])
 def test_rule(m, n, k, want):
     assert ops.prefill_path(m, SimpleNamespace(n=n, k=k, packed=None, packed_v3=None, packed_mma=object())) is want
+
+
+def test_results_are_plain_tensors(monkeypatch):
+    class Sub(torch.Tensor):
+        pass
+    monkeypatch.setattr(_native, "torch", torch)
+    x = torch.randn(3, 8).half()
+    for v in (x, x.as_subclass(Sub), torch.nn.Parameter(x)):
+        y = _native._output_rows(v, 3, 5)
+        assert type(y) is torch.Tensor and y.shape == (3, 5) and y.dtype is torch.float16 and not y.requires_grad
