@@ -367,8 +367,8 @@ hipError_t launch_prefill(const GemvArgs& a, const PrefillPlan& p, uint32_t* ctr
 // to 2048 rows of 12 Qwen2.5-0.5B .. 7B projections, 1 to 8 splits; the fit's error is 10-15%); the cheapest plan by it
 // is 2.5% slower than the sweep's best on average and 26% at worst. `alone` of the 64-row shapes was raised from the fit's
 // 0.74 and 0.66 afterwards: a workgroup that has its CU to itself and walks all of K waits for its weights (0.86 .. 0.9 a
-// chunk), so two splits beat it (2048 x 2048 at 512 rows 17.0 -> 14.2, 2048 x 2560 at 300 17.0 -> 14.2, 3584 x 4608 at 300
-// 28.0 -> 23.6, 1536 x 2048 at 400 13.0 -> 11.7).
+// chunk), so two splits beat it (2048 x 2048 at 512 rows 17.0 -> 14.2, 2048 x 2560 at 300 17.0 -> 14.2, 3584 x 4608 at 333
+// 28.1 -> 25.1, 3584 x 3584 at 400 27.8 -> 24.9, 1536 x 2048 at 512 13.0 -> 12.1).
 struct PrefillShape {
   int MT, PT, groups;
   float base, alone, each, split, per_mb;
@@ -376,8 +376,8 @@ struct PrefillShape {
 constexpr PrefillShape kPrefillShapes[] = {
     {8, 2, 2, 4.8f, 1.20f, 0.93f, 4.4f, 0.30f},             // 128 activation rows x 128 weight rows
     {6, 4, 2, 6.8f, 1.41f, 1.25f, 6.9f, 0.24f},             // 96 x 256
-    {4, 2, 4, 4.2f, 0.85f, 0.56f, 2.7f, 0.31f},             // 64 x 128
-    {4, 1, 4, 2.5f, 0.85f, 0.385f, 2.0f, 0.38f},            // 64 x 64
+    {4, 2, 4, 4.2f, 0.88f, 0.56f, 2.7f, 0.31f},             // 64 x 128
+    {4, 1, 4, 2.5f, 0.88f, 0.385f, 2.0f, 0.38f},            // 64 x 64
 };
 constexpr int kCUs = 256;
 
