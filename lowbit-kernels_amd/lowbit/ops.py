@@ -205,14 +205,15 @@ def prefill(x, wq):
 
 
 def _prefill_without_blas(m, wq):
-    """The part of prefill_path that holds whatever is asked of x: the rest keeps dequantize + BLAS for calls that
-    torch differentiates or transforms (_plain)."""
+    """The part of prefill_path that holds whatever is asked of x and the bias: the rest keeps dequantize + BLAS for
+    calls that torch differentiates or transforms (_plain)."""
     return (wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS
             or (m <= AUTO_PREFILL_NARROW_ROWS and wq.n <= AUTO_PREFILL_NARROW and wq.k <= AUTO_PREFILL_NARROW))
 
 
 def prefill_path(m, wq):
-    """True when linear() sends m rows to the int4 prefill GEMM rather than dequantize + BLAS (auto routing only)."""
+    """True when linear() sends m rows to the int4 prefill GEMM rather than dequantize + BLAS (auto routing only; the
+    calls that _plain refuses keep BLAS where _prefill_without_blas does not hold)."""
     if auto_version(m, wq) is not None or wq.packed_mma is None:
         return False
     if _prefill_without_blas(m, wq):
@@ -225,14 +226,19 @@ def prefill_path(m, wq):
     return tiles > 256 and tiles < AUTO_PREFILL_FILL * 256 * -(-tiles // 256)
 
 
-def _plain(x):
-    """True when x is an fp16 matrix of which only the values matter: no gradient, autocast, forward-mode level, function
-    transform, trace, tensor subclass or third dimension that the BLAS GEMM, a torch operator, would serve and a kernel
-    call would not."""
-    return (type(x) in (torch.Tensor, torch.nn.Parameter) and x.dim() == 2 and x.dtype is torch.float16
-            and not (x.requires_grad and torch.is_grad_enabled()) and not torch.is_autocast_enabled()
-            and torch.autograd.forward_ad._current_level < 0 and not torch.jit.is_tracing()
-            and not torch._C._functorch.is_functorch_wrapped_tensor(x))
+def _values_only(t):
+    """True when only t's values matter: no gradient, function transform or tensor subclass that a torch operator would
+    serve and a kernel call, which takes the address, would not."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and not (t.requires_grad and torch.is_grad_enabled())
+            and not torch._C._functorch.is_functorch_wrapped_tensor(t))
+
+
+def _plain(x, bias=None):
+    """True when x is an fp16 matrix, and bias a vector, of which only the values matter, outside autocast, forward-mode
+    levels and traces: what the BLAS GEMM and the add after it, torch operators, would serve beyond that is not asked."""
+    return (_values_only(x) and x.dim() == 2 and x.dtype is torch.float16 and (bias is None or _values_only(bias))
+            and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0
+            and not torch.jit.is_tracing())
 
 
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
@@ -246,6 +252,7 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     m = x.shape[0]
     if m == 0:
         return x.new_empty(0, wq.n)
+    given = bias                              # the caller's: a conversion below may leave its type behind
     if bias is not None:                      # one bias for every route: fp16 [N] on x's device
         if bias.numel() != wq.n:
             raise ValueError(f"bias must hold N={wq.n} values, got shape {list(bias.shape)}")
@@ -263,7 +270,7 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
         return ext().w4_linear_fused(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias)
     if v is not None:
         y = gemv(x, wq, v)
-    elif version == 0 and prefill_path(m, wq) and (_prefill_without_blas(m, wq) or _plain(x)):
+    elif version == 0 and prefill_path(m, wq) and (_prefill_without_blas(m, wq) or _plain(x, given)):
         if bias is not None:
             return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias)
         y = prefill(x, wq)

@@ -24,7 +24,9 @@ def layer(monkeypatch):
         return call
     monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq: x.detach() @ w.t()))
     monkeypatch.setattr(ops, "dequant", fake("dequant", lambda *a: w))
-    wq = SimpleNamespace(n=N, k=K, packed=None, packed_v3=None, packed_mma=object())
+    monkeypatch.setattr(ops, "ext", lambda: SimpleNamespace(w4_gemm_prefill=fake(
+        "prefill+bias", lambda x, p, s, g, epilogue, bias: (x.detach() @ w.t()).add_(bias.detach()))))
+    wq = SimpleNamespace(n=N, k=K, packed=None, packed_v3=None, packed_mma=object(), scales=None, group=128)
     assert ops.prefill_path(M, wq) and not ops._prefill_without_blas(M, wq)
     return wq, w, taken
 
@@ -57,6 +59,34 @@ def test_transformed_calls_keep_blas(layer):
     x3 = torch.randn(M, 2, K).half()
     assert near(ops.linear(x3, wq), x3 @ w.t())
     assert taken == ["dequant"] * 4
+
+
+def test_the_bias_counts_as_x_does(layer):
+    wq, w, taken = layer
+    x = torch.randn(M, K).half()
+    b = torch.randn(N).half()
+    with torch.no_grad():
+        ops.linear(x, wq, bias=b.clone().requires_grad_())
+    for plain in (b, torch.nn.Parameter(b, requires_grad=False), b.float()):
+        assert near(ops.linear(x, wq, bias=plain), x @ w.t() + b)
+    assert taken == ["prefill+bias"] * 4
+    taken.clear()
+    for bias in (torch.nn.Parameter(b.clone()), b.float().requires_grad_(), b.view(1, N).clone().requires_grad_()):
+        y = ops.linear(x, wq, bias=bias)
+        assert y.requires_grad
+        y.float().sum().backward()
+        assert torch.equal(bias.grad.view(N).float(), torch.full((N,), float(M)))
+    got = torch.func.grad(lambda a: ops.linear(x, wq, bias=a).float().sum())(b)
+    assert torch.equal(got, torch.full((N,), float(M)).half())
+    with fwad.dual_level():
+        t = torch.randn(N).half()
+        out = ops.linear(x, wq, bias=fwad.make_dual(b.clone(), t))
+        assert torch.equal(fwad.unpack_dual(out).tangent, t.expand(M, N))
+
+    class Sub(torch.Tensor):
+        pass
+    assert type(ops.linear(x, wq, bias=b.as_subclass(Sub))) is Sub
+    assert taken == ["dequant"] * 6
 
 
 @pytest.mark.parametrize("m,n,k,want", [
