@@ -235,10 +235,11 @@ def _values_only(t):
 
 def _plain(x, bias=None):
     """True when x is an fp16 matrix, and bias a vector, of which only the values matter, outside autocast, forward-mode
-    levels and traces: what the BLAS GEMM and the add after it, torch operators, would serve beyond that is not asked."""
+    levels and traces: what the BLAS GEMM and the add after it, torch operators, would serve beyond that is not asked.
+    x must also be where the kernel's 16-byte loads can read it (a contiguous x is passed as it is, any other copied)."""
     return (_values_only(x) and x.dim() == 2 and x.dtype is torch.float16 and (bias is None or _values_only(bias))
             and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0
-            and not torch.jit.is_tracing())
+            and not torch.jit.is_tracing() and (x.data_ptr() % 16 == 0 or not x.is_contiguous()))
 
 
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):

@@ -89,6 +89,19 @@ def test_the_bias_counts_as_x_does(layer):
     assert taken == ["dequant"] * 6
 
 
+def test_x_off_the_16_byte_grid_keeps_blas(layer):
+    """A contiguous view that starts on any fp16 element was served by the BLAS GEMM; the int4 GEMM refuses it."""
+    wq, w, taken = layer
+    x = torch.randn(M, K).half()
+    buf = torch.empty(M * K + 8, dtype=torch.float16)
+    for off in (1, 2, 4, 8):
+        at = buf[off:off + M * K].view(M, K).copy_(x)
+        assert at.is_contiguous() and near(ops.linear(at, wq), x @ w.t())
+    wide = torch.empty(M, K + 1, dtype=torch.float16)[:, 1:].copy_(x)        # copied to its own, aligned, memory
+    assert near(ops.linear(wide, wq), x @ w.t())
+    assert taken == ["dequant"] * 3 + ["prefill"] * 2
+
+
 @pytest.mark.parametrize("m,n,k,want", [
     (512, 8192, 2048, True), (513, 8192, 2048, False), (513, 4096, 8960, True), (1024, 8193, 2048, True),
     (1025, 4096, 8960, False), (1024, 4097, 2048, False), (1400, 22016, 2048, True), (1400, 18944, 3584, False),
