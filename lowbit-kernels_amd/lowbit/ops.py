@@ -233,13 +233,22 @@ def _values_only(t):
             and not torch._C._functorch.is_functorch_wrapped_tensor(t))
 
 
+def _modes():
+    """True under a torch dispatch or function mode, such as a FLOP counter, which sees the BLAS GEMM but no kernel call.
+    The default device is a function mode too, and one that leaves products alone."""
+    return (torch._C._len_torch_dispatch_stack() > 0
+            or (torch._C._len_torch_function_stack() > 0
+                and any(type(m) is not torch.utils._device.DeviceContext
+                        for m in torch.overrides._get_current_function_mode_stack())))
+
+
 def _plain(x, bias=None):
     """True when x is an fp16 matrix, and bias a vector, of which only the values matter, outside autocast, forward-mode
-    levels and traces: what the BLAS GEMM and the add after it, torch operators, would serve beyond that is not asked.
+    levels, traces and modes: what the BLAS GEMM and the add after it, torch operators, would serve beyond that is not asked.
     x must also be where the kernel's 16-byte loads can read it (a contiguous x is passed as it is, any other copied)."""
     return (_values_only(x) and x.dim() == 2 and x.dtype is torch.float16 and (bias is None or _values_only(bias))
             and not torch.is_autocast_enabled() and torch.autograd.forward_ad._current_level < 0
-            and not torch.jit.is_tracing() and (x.data_ptr() % 16 == 0 or not x.is_contiguous()))
+            and not torch.jit.is_tracing() and not _modes() and (x.data_ptr() % 16 == 0 or not x.is_contiguous()))
 
 
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):

@@ -6,6 +6,7 @@ from types import SimpleNamespace
 import pytest
 import torch
 import torch.autograd.forward_ad as fwad
+import torch.utils.flop_counter
 
 from lowbit import _native, ops
 
@@ -100,6 +101,26 @@ def test_x_off_the_16_byte_grid_keeps_blas(layer):
     wide = torch.empty(M, K + 1, dtype=torch.float16)[:, 1:].copy_(x)        # copied to its own, aligned, memory
     assert near(ops.linear(wide, wq), x @ w.t())
     assert taken == ["dequant"] * 3 + ["prefill"] * 2
+
+
+def test_calls_under_a_mode_keep_blas(layer):
+    wq, w, taken = layer
+    x = torch.randn(M, K).half()
+    with torch.utils.flop_counter.FlopCounterMode(display=False) as count:
+        ops.linear(x, wq)
+    assert count.get_total_flops() == 2 * M * N * K
+
+    class Mode(torch.overrides.TorchFunctionMode):
+        seen = 0
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            Mode.seen += func is torch.nn.functional.linear
+            return func(*args, **(kwargs or {}))
+    with Mode():
+        ops.linear(x, wq)
+    with torch.device("cpu"):
+        ops.linear(x, wq)
+    assert Mode.seen == 1 and taken == ["dequant", "dequant", "prefill"]
 
 
 @pytest.mark.parametrize("m,n,k,want", [
