@@ -258,15 +258,21 @@ def _output_rows(x, m, n):
     return torch.empty((m, n), dtype=torch.float16, device=x.device)
 
 
-def _launch(index, call, nbytes=0):
+def _launch(index, call, nbytes=0, own=False):
     """call(stream, workspace address, workspace bytes) on GPU `index`, made current for the call, with that GPU's current
     stream and its workspace of `nbytes` (0: none); raises on a non-zero status. The launch path of the projections: the
-    current device and stream come from torch's plain getters, as integers."""
+    current device and stream come from torch's plain getters, as integers. own: a call that is being captured takes a
+    workspace of its graph's memory, its counters cleared in the graph, rather than the stream's, which graphs captured on
+    one stream would share (they may then run at the same time)."""
     if torch._C._cuda_getDevice() != index:
         with torch.cuda.device(index):
-            return _launch(index, call, nbytes)
+            return _launch(index, call, nbytes, own)
     stream = torch._C._cuda_getCurrentRawStream(index)
-    if nbytes:
+    if own and torch.cuda.is_current_stream_capturing():
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=torch.device("cuda", index))
+        ws[:WORKSPACE_COUNTER_BYTES].zero_()
+        rc = call(stream, ws.data_ptr(), nbytes)
+    elif nbytes:
         ws = _WORKSPACES.get((index, stream or None, nbytes, ""))   # workspace()'s key
         if ws is None:
             ws = workspace(torch.device("cuda", index), ctypes.c_void_p(stream), nbytes)
@@ -390,15 +396,16 @@ class NativeExt:
             raise RuntimeError("out must be a contiguous float16 [M, N] (or [M, N/2] for silu-mul) tensor")
         return out
 
-    def w4_gemm_prefill(self, x, w, s, group, epilogue=EPI_STORE, aux=None, out=None):
+    def w4_gemm_prefill(self, x, w, s, group, epilogue=EPI_STORE, aux=None, out=None, own_workspace=False):
         """x [M, K] (any M, meant for M > 64) times the MFMA-layout weight, int4 read directly, with the epilogue
-        fused into the store; returns y ([M, N], or [M, N / 2] for EPI_SILU_MUL)."""
+        fused into the store; returns y ([M, N], or [M, N / 2] for EPI_SILU_MUL). own_workspace: a captured call keeps
+        its split-K partials in its graph's memory (_launch)."""
         m, n, k, index = _check_tensors(x, w, s, group)
         y = self._output(x, m, n, epilogue, out)
         _check_epilogue(epilogue, aux, m, n, x.device)
         _launch(index, lambda stream, ws, nbytes: self.lib.lowbit_w4_gemm_prefill(
             x.data_ptr(), w.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, group, int(epilogue),
-            aux.data_ptr() if aux is not None else None, ws, nbytes, stream), PREFILL_WORKSPACE_BYTES)
+            aux.data_ptr() if aux is not None else None, ws, nbytes, stream), PREFILL_WORKSPACE_BYTES, own_workspace)
         return y
 
     def rmsnorm(self, x, weight, eps, out=None):

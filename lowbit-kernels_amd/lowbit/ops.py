@@ -196,12 +196,12 @@ def auto_version(m, wq):
     return None
 
 
-def prefill(x, wq):
+def prefill(x, wq, own_workspace=False):
     """x [M, K] times an mma-layout weight with the int4-direct prefill GEMM (any M; fp32 accumulation of exactly the
-    dequantized fp16 weights, as dequantize + BLAS computes)."""
+    dequantized fp16 weights, as dequantize + BLAS computes). own_workspace: see w4_gemm_prefill."""
     if wq.packed_mma is None:
         raise ValueError("the prefill GEMM reads packed_mma, which this W4Weight does not keep")
-    return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group)
+    return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, own_workspace=own_workspace)
 
 
 def _prefill_without_blas(m, wq):
@@ -281,9 +281,12 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     if v is not None:
         y = gemv(x, wq, v)
     elif version == 0 and prefill_path(m, wq) and (_prefill_without_blas(m, wq) or _plain(x, given)):
+        # beyond _prefill_without_blas, calls captured on one stream share no scratch, as BLAS calls do not
+        own = not _prefill_without_blas(m, wq)
         if bias is not None:
-            return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias)
-        y = prefill(x, wq)
+            return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias,
+                                         own_workspace=own)
+        y = prefill(x, wq, own)
     else:
         y = torch.nn.functional.linear(x, dequant(wq, "mma" if wq.packed_mma is not None else "canonical"))
     return y.add_(bias) if bias is not None else y

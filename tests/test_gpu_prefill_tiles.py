@@ -59,3 +59,37 @@ def test_linear_agrees_on_both_prefill_routes(cuda, m, k, n):
     y = ops.linear(x, wq)
     assert_rounds(y, x.double() @ ops.dequant(wq, "mma").double().t())
     assert torch.equal(ops.linear(x, wq, bias=bias), y + bias)
+
+
+def test_captured_calls_share_no_scratch(cuda):
+    """Calls above AUTO_PREFILL_ROWS rows, with K split over workgroups, captured on one stream into graphs that are then
+    replayed at the same time on two streams, between eager calls: every replay gives the eager result. The stream has
+    captured before it has run any, and its first eager call comes after that."""
+    wq, *_, gen = make_weight(11008, 2048, 5, layouts=("mma",), sd=0.02)
+    bias = torch.randn(2048, generator=gen).half().cuda()
+    xs = [torch.randn(600, 11008, generator=gen).half().cuda() for _ in range(2)]
+    assert ops.prefill_path(600, wq) and not ops._prefill_without_blas(600, wq)
+    want = [ops.linear(x, wq, bias=bias) for x in xs]
+    side = torch.cuda.Stream()
+    graphs, outs = [torch.cuda.CUDAGraph() for _ in xs], []
+    for g, x in zip(graphs, xs):
+        with torch.cuda.graph(g, stream=side):
+            for _ in range(4):
+                y = ops.linear(x, wq, bias=bias)
+            outs.append(y)
+    with torch.cuda.stream(side):
+        eager = ops.linear(xs[0], wq, bias=bias)
+    torch.cuda.synchronize()
+    assert torch.equal(eager, want[0])
+    streams = [torch.cuda.Stream() for _ in xs]
+    for _ in range(3):
+        for y in outs:
+            y.zero_()
+        torch.cuda.synchronize()
+        for g, s in zip(graphs, streams):
+            with torch.cuda.stream(s):
+                g.replay()
+        torch.cuda.synchronize()
+        for y, w in zip(outs, want):
+            assert torch.equal(y, w)
+        assert torch.equal(ops.linear(xs[1], wq, bias=bias), want[1])

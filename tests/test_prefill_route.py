@@ -21,12 +21,12 @@ def layer(monkeypatch):
     def fake(name, result):
         def call(*args, **kwargs):
             taken.append(name)
-            return result(*args)
+            return result(*args, **kwargs)
         return call
-    monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq: x.detach() @ w.t()))
+    monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq, own: x.detach() @ w.t()))
     monkeypatch.setattr(ops, "dequant", fake("dequant", lambda *a: w))
     monkeypatch.setattr(ops, "ext", lambda: SimpleNamespace(w4_gemm_prefill=fake(
-        "prefill+bias", lambda x, p, s, g, epilogue, bias: (x.detach() @ w.t()).add_(bias.detach()))))
+        "prefill+bias", lambda x, p, s, g, epilogue, bias, **own: (x.detach() @ w.t()).add_(bias.detach()))))
     wq = SimpleNamespace(n=N, k=K, packed=None, packed_v3=None, packed_mma=object(), scales=None, group=128)
     assert ops.prefill_path(M, wq) and not ops._prefill_without_blas(M, wq)
     return wq, w, taken
