@@ -183,6 +183,14 @@ class FusedQwen2:
         self.k_cache.zero_()
         self.v_cache.zero_()
 
+    def _embedding(self, tokens):
+        """F.embedding. Up to 16 int64 ids through gather, where F.embedding picks a small-index kernel (12 us at 16 ids
+        against 5); gather takes a row's id once per column, which needs int64 (of int32 ids, which F.embedding takes
+        too, an expanded index reads the first alone on the CPU)."""
+        if tokens.dim() == 1 and tokens.shape[0] <= 16 and tokens.dtype is torch.int64:
+            return torch.gather(self.embed, 0, tokens[:, None].expand(tokens.shape[0], self.hidden))
+        return F.embedding(tokens, self.embed)
+
     def head_picks(self):
         """True when a one-row step's head can take the greedy pick along (lowbit_f16_gemv_pick)."""
         return self.hidden * 2 <= 65536
@@ -210,8 +218,8 @@ class FusedQwen2:
         [M, hidden] when the caller already holds them (it becomes the residual stream, overwritten)."""
         ext = ops.ext()
         m = tokens.shape[0]
-        if h is None:                                         # (up to 16 tokens F.embedding picks a small-index kernel, 12
-            h = torch.gather(self.embed, 0, tokens[:, None].expand(m, self.hidden))   # us at 16 against 5; same checks)
+        if h is None:
+            h = self._embedding(tokens)
         xn = torch.empty_like(h)
         q = torch.empty(m, self.hq, self.head_dim, dtype=torch.float16, device=h.device)
         attn = torch.empty(m, self.hq * self.head_dim, dtype=torch.float16, device=h.device)
