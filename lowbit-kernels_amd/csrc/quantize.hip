@@ -99,7 +99,8 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
 // (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).
 // It is the correctly rounded quotient: the scale is an fp16 value, so its 11 bits make r exact and keep v / scale at least
 // 2^-12 ulp away from every rounding boundary, far more than the ~2^-22 ulp that y's error can move the sum by; an infinite
-// scale, whose reciprocal says nothing, takes the division itself.
+// scale, whose reciprocal says nothing, and a group whose largest quotient overflows (a clip factor near 0 on weights near
+// fp32's largest; q0 would be infinite and r not a number) take the division itself.
 // Bound: vector instructions (8 per value and candidate; the division took ~10 by itself). 11008 x 2048 fp16, 11
 // candidates, MI355X: quantize_kernel 208 us, 72 here.
 template <int kDtype>
@@ -143,11 +144,11 @@ __global__ __launch_bounds__(256) void quantize_groups(const void* __restrict__ 
   for (int e = 0; e < 8; e += 2) amax = fmaxf(amax, fmaxf(fabsf(v[e]), fabsf(v[e + 1])));
   amax = over_group(amax, [](float a, float b) { return fmaxf(a, b); });
   auto quantize8 = [&](float scf, auto each) {              // each(e, quantized value), e = 0..7
-    if (__any(__builtin_isinf(scf))) {
+    const float y = 1.0f / scf;
+    if (__any(__builtin_isinf(scf) || __builtin_isinf(amax * y))) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) each(e, quantize_one(v[e], scf));
     } else {
-      const float y = 1.0f / scf;
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float q0 = v[e] * y, r = fmaf(-q0, scf, v[e]);

@@ -48,3 +48,15 @@ def test_same_bits_on_hard_values(cuda, dtype):
         for group in (32, 64, 128):
             for grid in (None, CLIP):
                 both(w.to(dtype).contiguous(), group, grid)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_same_bits_where_quotients_overflow(cuda, dtype):
+    """Clip factors near 0 on weights near fp32's largest value: finite scales whose quotients pass fp32's range."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    w = (torch.randn(64, 256, generator=g, device="cuda").clamp(-3, 3) * 1e38).to(dtype)
+    assert bool(torch.isfinite(w).all())
+    for group in (32, 64, 128):
+        for grid in ((1e-38,), (1e-37, 3e-38, 1e-38, 3e-39), (2e-38, 1.0), (0.0,)):
+            both(w, group, grid)
+        both(torch.cat([w[:3], w[3:6] * 1e-38]), group, (1e-38, 1.0))
