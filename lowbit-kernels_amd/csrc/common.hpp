@@ -211,8 +211,10 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 // carries the wave-uniform `lds`). Written as inline asm, so the compiler neither inserts waits for it nor holds LDS
 // accesses back behind it: the caller counts these loads itself (lds_wait_read16, lds_wait_barrier). Vector-memory
 // operations of one wave complete in issue order, so "at most N outstanding" means everything but the newest N has
-// landed; a load of the compiler's issued later only makes such a wait longer, never short. m0 is otherwise unused
-// by the kernels that call this (gfx9 LDS instructions do not read it).
+// landed. A load of the compiler's that the caller does not count only makes such a wait longer; one that it does count
+// as newer than the loads waited for must have been issued, so its value must be used on every path on which the count
+// is relied on (the compiler drops a load whose value is not). m0 is otherwise unused by the kernels that call this
+// (gfx9 LDS instructions do not read it).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t r, int voffset, uint32_t lds) {

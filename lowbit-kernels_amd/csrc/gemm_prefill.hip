@@ -125,8 +125,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   const uint8_t* xtile = reinterpret_cast<const uint8_t*>(x) + (size_t)m0 * K * 2;
   const int ustep = kThreads / 8 * K;                       // bytes from one u's rows to the next one's
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(xtile, (uint32_t)(16 * MT * K * 2));
-  auto issue_x = [&](int b, int chunk) __attribute__((always_inline)) {   // chunk of x straight into LDS buffer b
-    const int c = min(chunk, ce - 1);
+  auto issue_x = [&](int b, int c) __attribute__((always_inline)) {   // chunk c of x straight into LDS buffer b
     if (!ragged) {
       int at = 256 * c;
 #pragma unroll
@@ -168,7 +167,9 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   // buffer j % 2, its weights in slot j % 2. The slot is refilled two chunks ahead when its last k-step has been decoded;
   // before the last group, when every B fragment of the chunk has been read, one barrier makes the next chunk's x
   // visible (the wait leaves the 2 PT newer weight loads in flight) and frees this chunk's buffer for the x two chunks
-  // ahead. (Left to itself hipcc waits for every pair of fragment reads right after issuing it.)
+  // ahead. The count relies on those loads, which are the compiler's own, being there: they are while the chunk they
+  // fetch is consumed, and where it is past the range (the last two chunks), the wait is for everything. (Left
+  // to itself hipcc waits for every pair of fragment reads right after issuing it.)
   constexpr int GP = MT / 2, DPG = (PT + GP - 1) / GP;      // groups per k-step, decodes per group
   f16x8 a[2][PT], bx[2][2];
   auto chunk = [&](int j, auto slot) __attribute__((always_inline)) {
@@ -178,8 +179,12 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
       constexpr bool last = g + 1 == 4 * GP;
       if constexpr (g == 3 * GP) issue_w(d, cb + j + 2);
       if constexpr (last) {
-        lds_wait_barrier<2 * PT>();
-        issue_x(d, cb + j + 2);
+        if (j + 2 < nsteps) {
+          lds_wait_barrier<2 * PT>();
+          issue_x(d, cb + j + 2);
+        } else {
+          lds_wait_barrier<0>();
+        }
       }
 #pragma unroll
       for (int e = 0; e < 2; ++e)
@@ -204,8 +209,12 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   issue_w(0, cb);
   issue_x(0, cb);
   issue_w(1, cb + 1);
-  issue_x(1, cb + 1);
-  lds_wait_barrier<2 * PT + XP>();                          // chunk 0 of x has landed
+  if (nsteps > 1) {
+    issue_x(1, cb + 1);
+    lds_wait_barrier<2 * PT + XP>();                        // chunk 0 of x has landed
+  } else {
+    lds_wait_barrier<0>();
+  }
 #pragma unroll
   for (int e = 0; e < 2; ++e) bx[0][e] = *reinterpret_cast<const f16x8*>(smem + 4096 * e + xrd[0]);
 #pragma unroll
