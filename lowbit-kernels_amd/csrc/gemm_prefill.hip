@@ -296,6 +296,7 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   // 2048 x 16384 outputs the stores alone took 35 us a round of tiles). Rows are padded by 32 bytes: the 16 rows x 32
   // bytes of a wave's write then meet different banks.
   constexpr int kPitch = 2 * kRows + 32;
+  typedef f16 row8 __attribute__((ext_vector_type(8), aligned(2)));   // 8 values of a row, at any 2-byte address
   lds_barrier();                                            // (s_last has been read)
 #pragma unroll
   for (int i = 0; i < PT; ++i)
@@ -309,7 +310,6 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
   if (epi.mode == kEpiSiluMul) {                            // 8 outputs from a 16-row tile's 8 gate and 8 up values (all
     constexpr int kPcs = kRows / 16;                        // lanes busy: in the registers' layout half of them hold up)
     const int ny = N / 2;                                   // (N % 16 == 0)
-    const bool vec = (reinterpret_cast<uintptr_t>(y) & 15) == 0;
     for (int p = tid; p < 16 * MT * kPcs; p += kThreads) {
       const int row = p / kPcs, m = m0 + row, n = n0 / 2 + 8 * (p % kPcs);
       if (m >= M || n >= ny) continue;
@@ -322,39 +322,32 @@ __global__ __launch_bounds__(256, 2) void gemm_prefill(
         o[e] = as_u32(f16x2{silu_mul((float)g2[0], (float)u2[0]), silu_mul((float)g2[1], (float)u2[1])});
       }
       f16* dst = y + (size_t)m * ny + n;
-      if (vec) {
-        *reinterpret_cast<u32x4*>(dst) = o;
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dst[e] = as_f16x2(o[e >> 1])[e & 1];
-      }
+      *reinterpret_cast<row8*>(dst) = __builtin_bit_cast(f16x8, o);
     }
     return;
   }
+  // 8 values a piece, at any 2-byte address (global memory takes dwordx4 accesses at those), then the values past the last
+  // whole piece of the rows. Single values wherever a piece is not 16-byte aligned, as this kernel stored them before: 333
+  // rows of 2048 x 11004 37 us, 32.3 now; 512 of 3584 x 18941 85 -> 77; 2048 of 1024 x 4100 37 -> 26 (a width of 11008
+  // 32.3 both ways). The rows' ends inside the loop, with a residual: 40.5 us where they now take 36.
   constexpr int kPcs = kRows / 8;
   const bool aux = epi.mode == kEpiBias || epi.mode == kEpiResidual;
-  const bool vec = (N & 7) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0 &&
-                   (!aux || (reinterpret_cast<uintptr_t>(epi.aux) & 15) == 0);
+  auto add_at = [&](int m, int n) { return epi.mode == kEpiBias ? epi.aux + n : epi.aux + (size_t)m * N + n; };
   for (int p = tid; p < 16 * MT * kPcs; p += kThreads) {
     const int row = p / kPcs, m = m0 + row, n = n0 + 8 * (p % kPcs);
-    if (m >= M || n >= N) continue;
-    const u32x4 v = *reinterpret_cast<const u32x4*>(smem + row * kPitch + 16 * (p % kPcs));
-    f16* dst = y + (size_t)m * N + n;
-    const f16* add = epi.mode == kEpiBias ? epi.aux + n : epi.aux + (size_t)m * N + n;
-    if (vec) {
-      u32x4 o = v;
-      if (aux) {
-        const u32x4 t = *reinterpret_cast<const u32x4*>(add);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = as_u32(as_f16x2(v[e]) + as_f16x2(t[e]));
-      }
-      *reinterpret_cast<u32x4*>(dst) = o;
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (n + e < N) dst[e] = aux ? as_f16x2(v[e >> 1])[e & 1] + add[e] : as_f16x2(v[e >> 1])[e & 1];
-    }
+    if (m >= M || n + 8 > N) continue;
+    f16x8 v = *reinterpret_cast<const f16x8*>(smem + row * kPitch + 16 * (p % kPcs));
+    if (aux) v += *reinterpret_cast<const row8*>(add_at(m, n));
+    *reinterpret_cast<row8*>(y + (size_t)m * N + n) = v;
   }
+  const int nw = N & ~7;
+  if (nw < N && n0 + kRows > nw)
+    for (int p = tid; p < 16 * MT * 8; p += kThreads) {
+      const int row = p >> 3, m = m0 + row, n = nw + (p & 7);
+      if (m >= M || n >= N) continue;
+      const f16 v = *reinterpret_cast<const f16*>(smem + row * kPitch + 2 * (n - n0));
+      y[(size_t)m * N + n] = aux ? v + *add_at(m, n) : v;
+    }
 }
 
 namespace {

@@ -18,7 +18,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("m,k,n", [
     (64, 128, 64), (65, 128, 250), (95, 384, 257), (96, 640, 1000), (97, 256, 1004), (127, 1152, 998), (128, 896, 4864),
     (129, 2048, 2050), (191, 11008, 130), (192, 8960, 1536), (193, 4096, 72), (255, 1536, 8961), (257, 128, 8960),
-    (700, 2048, 2560), (385, 1024, 11008), (1025, 640, 4099), (640, 384, 22016)])
+    (65, 128, 5), (333, 256, 11004), (333, 256, 11003), (700, 2048, 2560), (385, 1024, 11008), (1025, 640, 4099), (640, 384, 22016)])
 def test_tile_edges(cuda, m, k, n):
     wq, *_, gen = make_weight(k, n, m + k + n, layouts=("mma",), sd=0.02)
     x = torch.randn(m, k, generator=gen).half().cuda()
