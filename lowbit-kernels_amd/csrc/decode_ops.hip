@@ -863,12 +863,18 @@ constexpr int kHeadRows = 2;                                // RW: rows per wave
 // Bound: HBM. 151936 x 2048 head (622 MB, 3 cold copies), MI355X, us (direct fragments -> this; hipBLASLt): 16 rows
 // 134 -> 104 (205), 32 rows 145 -> 114 (147), 48 rows 156 -> 133 (144), 64 rows 166 -> 144 (154); one more slot at 16
 // rows, which costs the second workgroup per CU, 110.
-constexpr int f16w_slots(int MT) { return MT == 1 ? 4 : 3; }   // (80 KB of LDS: two workgroups per CU)
+// Slots: two workgroups share a CU at up to 32 rows (80 and 72 KB of LDS), one at more (84 and 96 KB). There, weights of
+// more than one workgroup a CU whose chunks are few, so that the pipeline's start and end count, take two slots and so
+// two workgroups a CU (f16w_short). us at 48 and 64 rows, two slots / three: 151936 x 128 15.6 and 17.8 / 24.0 and 27.2, x
+// 512 34.8 and 39.1 / 44.0 and 49.1, x 1024 62 and 67 / 69 and 79, x 1536 92 and 100 / 100 and 111, x 2048 134 and 141 / 130
+// and 142; 18944 x 1024 11.6 and 12.7 / 13.2 and 14.9; but 2048 x 2048 13.0 and 13.6 / 10.0 and 11.4.
+constexpr int f16w_slots(int MT) { return MT == 1 ? 4 : 3; }
+constexpr bool f16w_short(int N, int K) { return N > 64 * 256 && K <= 1536; }
 constexpr int f16w_swz(int r) { return ((r & 3) << 2) | (r >> 2); }
-template <int MT>
+template <int MT, int D>
 __global__ __launch_bounds__(256) void gemm_f16w_rows_kernel(const f16* __restrict__ x, const f16* __restrict__ w,
                                                              f16* __restrict__ y, int M, int N, int K) {
-  constexpr int D = f16w_slots(MT), kTile = 16 * 256;           // bytes of 16 rows of a chunk
+  constexpr int kTile = 16 * 256;                           // bytes of 16 rows of a chunk
   constexpr int kSlot = (4 + MT) * kTile;                   // a chunk: the waves' W tiles, then x
   constexpr int kLoads = 4 + MT;                            // a wave's loads of a chunk
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -944,20 +950,26 @@ __global__ __launch_bounds__(256) void gemm_f16w_rows_kernel(const f16* __restri
   }
 }
 
-template <int MT>
+template <int MT, int D>
 hipError_t launch_f16w_rows(const f16* x, const f16* w, f16* y, int M, int N, int K, hipStream_t st) {
-  constexpr size_t lds = (size_t)f16w_slots(MT) * (4 + MT) * 16 * 256;
-  static const hipError_t attr = allow_lds(gemm_f16w_rows_kernel<MT>, lds);
-  if (attr != hipSuccess) return attr;
-  return launch(gemm_f16w_rows_kernel<MT>, dim3((unsigned)((N + 63) / 64)), dim3(256), lds, st, x, w, y, M, N, K);
+  constexpr size_t lds = (size_t)D * (4 + MT) * 16 * 256;
+  if (lds > 65536) {
+    static const hipError_t attr = allow_lds(gemm_f16w_rows_kernel<MT, D>, lds);
+    if (attr != hipSuccess) return attr;
+  }
+  return launch(gemm_f16w_rows_kernel<MT, D>, dim3((unsigned)((N + 63) / 64)), dim3(256), lds, st, x, w, y, M, N, K);
 }
 
 hipError_t gemm_f16w_rows_launch(const f16* x, const f16* w, f16* y, int M, int N, int K, hipStream_t st) {
   switch ((M + 15) / 16) {
-    case 1: return launch_f16w_rows<1>(x, w, y, M, N, K, st);
-    case 2: return launch_f16w_rows<2>(x, w, y, M, N, K, st);
-    case 3: return launch_f16w_rows<3>(x, w, y, M, N, K, st);
-    default: return launch_f16w_rows<4>(x, w, y, M, N, K, st);
+    case 1: return launch_f16w_rows<1, f16w_slots(1)>(x, w, y, M, N, K, st);
+    case 2: return launch_f16w_rows<2, f16w_slots(2)>(x, w, y, M, N, K, st);
+    case 3:
+      if (f16w_short(N, K)) return launch_f16w_rows<3, 2>(x, w, y, M, N, K, st);
+      return launch_f16w_rows<3, f16w_slots(3)>(x, w, y, M, N, K, st);
+    default:
+      if (f16w_short(N, K)) return launch_f16w_rows<4, 2>(x, w, y, M, N, K, st);
+      return launch_f16w_rows<4, f16w_slots(4)>(x, w, y, M, N, K, st);
   }
 }
 

@@ -196,18 +196,22 @@ class FusedQwen2:
         return self.hidden * 2 <= 65536
 
     def logits(self, xn, pick=None):
-        """The tied fp16 head: the library's fp16 GEMV for up to 32 rows, or 64 while hidden <= 2048 (against hipBLASLt,
-        3B head: 94 and 203 us at one row, 119 and 204 at 8, 104 and 205 at 16, 114 and 147 at 32, 144 and 154 at 64;
-        7B: 165 and 230 at 16, 181 and 248 at 32), hipBLASLt beyond (7B at 48 rows 212 and 200). pick = (tokens, positions[, out_tokens, out_count, h_next]),
-        one row (head_picks()): the GEMV also writes the greedy pick to tokens[0], advances positions[0] and, given
-        the rest, appends the pick to out_tokens and writes its embedding row to h_next (the next step's input)."""
+        """The tied fp16 head: the library's fp16 GEMV for up to 32 rows, or 64 while hidden <= 2048 on a vocabulary of
+        65536 or more (against hipBLASLt, 3B head: 94 and 203 us at one row, 119 and 204 at 8, 102 and 206 at 16, 106
+        and 145 at 32, 142 and 157 at 64; 151936 rows of 384 .. 1536 at 64: 33 and 41, 63 and 70 at 896, 100 and 112;
+        7B: 167 and 231 at 16, 179 and 247 at 32), hipBLASLt beyond (7B at 48 rows 213 and 205; 5120 at 48 289 and 276;
+        40000 x 1536 at 64, whose tiles end in a short round, 34 and 31). pick = (tokens, positions[, out_tokens,
+        out_count, h_next]), one row (head_picks()): the GEMV also writes the greedy pick to tokens[0], advances
+        positions[0] and, given the rest, appends the pick to out_tokens and writes its embedding row to h_next (the next
+        step's input)."""
         if pick is not None:
             more = {}
             if len(pick) > 2:
                 more = dict(out_tokens=pick[2], out_count=pick[3], embed=self.embed, h_out=pick[4])
             return ops.ext().f16_gemv_pick(xn, self.head, pick[0], pick[1], **more)
         m, k = xn.shape
-        if (m <= 8 and m * k * 2 <= 65536) or (m <= (64 if k <= 2048 else 32) and k % 128 == 0):
+        rows = 64 if k <= 2048 and self.head.shape[0] >= 65536 else 32
+        if (m <= 8 and m * k * 2 <= 65536) or (m <= rows and k % 128 == 0):
             return ops.ext().f16_gemv(xn, self.head)
         return F.linear(xn, self.head)
 

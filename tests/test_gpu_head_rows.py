@@ -1,5 +1,6 @@
 """The fp16-weight MFMA head kernel (lowbit_f16_gemv beyond 8 rows) where its ring and tiles can go wrong: fewer chunks of K
-than the ring holds, one more and many; 9, 16, 17, 33, 48, 49 and 64 rows; N beside multiples of 64, 16 and 4.
+than the ring holds, one more and many; 9, 16, 17, 33, 48, 49 and 64 rows; N beside multiples of 64, 16 and 4; the shorter
+ring of many-row, short-K weights.
 
 Bound: half an fp16 ulp of the result plus 2^-16 of the outputs' RMS for the fp32 sums, against the fp64 product."""
 import pytest
@@ -20,4 +21,10 @@ def test_head_rows(cuda, m, n, k):
     y = ops.ext().f16_gemv(x, w)
     assert_rounds(y, x.double() @ w.double().t())
     assert torch.equal(ops.ext().f16_gemv(x, w), y)
+
+
+@pytest.mark.parametrize("k", [128, 256, 384, 1536, 1664])
+@pytest.mark.parametrize("m,n", [(33, 16385), (48, 16450), (49, 16384), (64, 16516)])
+def test_head_rows_short_ring(cuda, m, n, k):
+    test_head_rows(cuda, m, n, k)
 
