@@ -464,9 +464,15 @@ __global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, 
 //   S^T = K Q^T: A = 32 keys x 16 dims from LDS, B = the wave's 32 rows (registers). Lane (j, h) holds row j's scores of
 //   keys 8 (v / 4) + 4 h + v % 4, v = 0..15: two lanes a row.
 //   Online softmax in base 2 against a reference that follows the running maximum only when a score exceeds it by more
-//   than kAttnLag (the weights then reach 2^kAttnLag at most), so that the 64 accumulator registers are rescaled in the
-//   first blocks only and no lane exchange is needed in the others. The weights are split into an fp16 head and an fp16
-//   remainder (to ~2^-22) as in attention_mfma.
+//   than a lag, so that the 64 accumulator registers are rescaled in the first blocks only and no lane exchange is
+//   needed in the others. The weights are split into an fp16 head and an fp16 remainder, together good to ~2^-22 of a
+//   weight while the remainder is a normal fp16 number and to half of fp16's smallest subnormal, 2^-25, below. They are
+//   therefore evaluated as 2^(score - reference + 15 - lag), with the maximum between 2^(15 - lag) and 2^15 (the factor
+//   cancels against their sum), so that what is cut off lies below 2^-39 of the largest weight at a lag of 1 and 2^-32 at
+//   8: a long tail of small weights keeps its sum. (Evaluated as 2^(score - reference), 64000 weights of 2^-26 vanished
+//   beside a weight of 1.) A lag of 1 rescales more often, which costs 1-2% with few rows and 13% with many (3000 tokens
+//   83 us against 73): the few rows whose other kernel is attention_kernel, with fp32 weights, take 1, the others, whose
+//   other kernel is attention_mfma, with weights of at most 1 and the same split, 8.
 //   O^T += V^T P^T: B = the weights as the lane holds them, i.e. contraction index 8 h + i of step s is key
 //   16 s + 8 (i / 4) + 4 h + i % 4; A = V^T from LDS by transposing reads (ds_read_b64_tr_b16).
 // K and V go from memory straight to LDS, one block ahead (K two: a block's scores are multiplied while the vector unit
@@ -480,7 +486,7 @@ __global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, 
 // MI355X, 16 query / 2 KV heads, us (attention_mfma -> this): 3000 tokens 285 -> 76, 700 tokens 32.5 -> 17.2, 300 tokens
 // 16.4 -> 11.4, 128 tokens 11.1 -> 8.9; 512 tokens on 4096 cached 204 -> 53, 128 on 8000 125 -> 39 (KG = 4; 70 and 49
 // with KG = 2); 28 / 4 heads, 2048 tokens 230 -> 63.
-constexpr float kAttnLag = 8.f;
+constexpr float kAttnLagFew = 1.f, kAttnLag = 8.f;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -566,6 +572,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
     const s16x4 c = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + at + 2048));
     return __builtin_bit_cast(f16x8, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
   };
+  const float lag = M * G < kAttnMfmaMinRows ? kAttnLagFew : kAttnLag;
   float ref = -INFINITY, lsum = 0.f;                          // reference (base 2), the lane's share of the weights' sum
   f32x16 o[4];
 #pragma unroll
@@ -593,7 +600,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
     float bm = st[0];
 #pragma unroll
     for (int v = 1; v < 16; ++v) bm = fmaxf(bm, st[v]);
-    if (__any(bm * c2 > ref + kAttnLag)) {                    // (uniform; either lane of a row)
+    if (__any(bm * c2 > ref + lag)) {                    // (uniform; either lane of a row)
       const float nm = fmaxf(ref, fmaxf(bm, __shfl_xor(bm, 32, 64)) * c2);   // -inf while the row has seen no key
       const float corr = nm == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(ref - nm);
       ref = nm;
@@ -601,7 +608,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) o[dt] *= corr;
     }
-    const float sub = ref == -INFINITY ? 0.f : ref;
+    const float sub = ref == -INFINITY ? 0.f : ref - (15.f - lag);
     const f32x16 sc = st;
     st = zero;
 #pragma unroll

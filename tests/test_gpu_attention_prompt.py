@@ -113,3 +113,26 @@ def test_prompt_attention_of_growing_scores(cuda):
     pos = torch.arange(960, 1024, device="cuda")
     check(q, k, v, pos, 128 ** -0.5, 1024)
     check(q, k.flip(1).contiguous(), v, pos, 128 ** -0.5, 1024)
+
+
+@pytest.mark.parametrize("m,drop,floor", [(1, 20.0, 39), (1, 24.0, 39), (1, 26.0, 39), (2, 26.0, 39), (16, 25.0, 32),
+                                          (64, 26.0, 32)])
+def test_long_tail_of_small_weights(cuda, m, drop, floor):
+    """One key of weight 1 and value 0 beside tens of thousands of weights of 2^-drop, whose sum alone makes the output.
+    Weights are good to 2^-39 of the largest below 32 rows per KV head and to 2^-32 from there on, 2^(drop - 39) or
+    2^(drop - 32) of these; the outputs are fp16."""
+    L, hq, hkv = 64000, 16, 2
+    q = torch.zeros(m, hq, 128, device="cuda").half()
+    q[..., 0] = 1
+    k = torch.zeros(hkv, L, 128, device="cuda").half()
+    k[:, 100, 0] = 128.0
+    v = (1 + 0.25 * torch.randn(hkv, L, 128, generator=torch.Generator(device="cuda").manual_seed(6), device="cuda")).half()
+    v[:, 100] = 0
+    scale = drop * math.log(2.0) / 128.0
+    pos = torch.full((m,), L - 1, device="cuda")
+    out = torch.empty(m, hq * 128, dtype=torch.float16, device="cuda")
+    ops.ext().attention(q, k, v, pos, out, hq, hkv, L, scale)
+    want = attend(q, k, v, pos, scale).view(m, -1)
+    assert bool((want > 1e-4).all())
+    err = (out.double() - want).norm() / want.norm()
+    assert err < BOUND + 2.0 ** (drop - floor), float(err)
