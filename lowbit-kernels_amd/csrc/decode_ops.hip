@@ -144,16 +144,15 @@ __device__ __forceinline__ float merge_partitions(__amdgpu_buffer_rsrc_t pr, int
   return num / den;
 }
 
+// the block bx of (token, head group)s, partition pid of P, whose partial goes to records `rec` ..
 template <int G, int KB>
-__global__ __launch_bounds__(G == 1 && KB == 32 ? 1024 : 512) void attention_kernel(
-    const f16* __restrict__ q, const f16* __restrict__ k_cache, const f16* __restrict__ v_cache,
-    const int64_t* __restrict__ pos, f16* __restrict__ out, int Hq, int Hkv, int L, float scale, int CH,
-    float* __restrict__ part) {
+__device__ __forceinline__ void attend_heads(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                             const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
+                                             f16* __restrict__ out, int Hq, int Hkv, int L, float scale, int CH,
+                                             float* __restrict__ part, uint8_t* smem, int bx, int pid, int P, size_t rec) {
   constexpr int NI = KB / 4;                                 // 16-byte loads per lane and step, per K and per V
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  args_in_sgprs(q, k_cache, v_cache, pos, out, Hq, Hkv, L, CH, part, (int)blockDim.x);
-  const int groups = Hq / G, P = gridDim.y, pid = blockIdx.y;
-  const int m = blockIdx.x / groups, h0 = (blockIdx.x % groups) * G, hk = h0 / (Hq / Hkv);
+  const int groups = Hq / G;
+  const int m = bx / groups, h0 = (bx % groups) * G, hk = h0 / (Hq / Hkv);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x >> 6;
   const int rg = lane >> 4, dl = (lane & 15) * 8;          // key row-group, first dim of the lane's slice
   const int64_t pm = pos[m];
@@ -237,8 +236,8 @@ __global__ __launch_bounds__(G == 1 && KB == 32 ? 1024 : 512) void attention_ker
     }
   }
   __syncthreads();
-  // partial of this block: [G][2 + D] floats (max, sum, then the unnormalized output), per (token, group, partition)
-  float* mine = part + (size_t)(blockIdx.x * P + pid) * G * kAttnRec;
+  // partial of this block: G records (max, sum, then the unnormalized output)
+  float* mine = part + rec * kAttnRec;
   for (int idx = threadIdx.x; idx < G * kHeadDim; idx += blockDim.x) {
     const int g = idx / kHeadDim, d = idx % kHeadDim;
     float gm = -INFINITY;
@@ -263,6 +262,17 @@ __global__ __launch_bounds__(G == 1 && KB == 32 ? 1024 : 512) void attention_ker
   }
 }
 
+template <int G, int KB>
+__global__ __launch_bounds__(G == 1 && KB == 32 ? 1024 : 512) void attention_kernel(
+    const f16* __restrict__ q, const f16* __restrict__ k_cache, const f16* __restrict__ v_cache,
+    const int64_t* __restrict__ pos, f16* __restrict__ out, int Hq, int Hkv, int L, float scale, int CH,
+    float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  args_in_sgprs(q, k_cache, v_cache, pos, out, Hq, Hkv, L, CH, part, (int)blockDim.x);
+  attend_heads<G, KB>(q, k_cache, v_cache, pos, out, Hq, Hkv, L, scale, CH, part, smem, blockIdx.x, blockIdx.y, gridDim.y,
+                      (size_t)(blockIdx.x * gridDim.y + blockIdx.y) * G);
+}
+
 // out[m][h][d] from the P <= kAttnMaxParts partials of attention_kernel or attention_mfma (merge_partitions), launched
 // after it
 __global__ __launch_bounds__(256) void attention_combine(const float* __restrict__ part, f16* __restrict__ out,
@@ -276,34 +286,69 @@ __global__ __launch_bounds__(256) void attention_combine(const float* __restrict
       (f16)merge_partitions(pr, b * P * G * kAttnRec + g * kAttnRec, G * kAttnRec, P, d);
 }
 
-// attention_combine for up to kAttnManyParts partitions: one block per (token, head), a thread per dim; the partitions'
-// weights exp(max - overall max) are evaluated once, a thread each, and shared through LDS (attention_combine has every
-// thread evaluate them all, which its at most 16 partitions hide behind one round trip)
-__global__ __launch_bounds__(kHeadDim) void attention_combine_many(const float* __restrict__ part, f16* __restrict__ out,
-                                                                   int Hq, int Hkv, int P) {
+// The key partitions of a call whose kernel is chosen on the device, by the keys attended (attention_select). The caller's
+// bound on the keys sizes the launch and may lie far above them (a captured step's bound is its cache), and a kernel that
+// is the better one on long contexts is not on the short ones at a conversation's start. The last token's position stands
+// for all; any choice is right for any positions. keys < from: attend_heads (by_head) or attend_mfma with up to `few`
+// partitions, else attend_prompt with up to `many`. The partials lie as [token][KV head][partition of `room`][head of the
+// KV head] records.
+struct AttnSplit {
+  int from, few, many, by_head, room;
+};
+// keys a partition of attend_heads takes, in four waves of 32
+__device__ __forceinline__ int attn_head_keys(int keys, int few) { return ((keys + few - 1) / few + 127) & ~127; }
+__device__ __forceinline__ int attn_parts(const AttnSplit& sp, int keys) {
+  if (keys >= sp.from) return min(sp.many, (keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys);
+  if (!sp.by_head) return keys <= kAttnMinKeys ? 1 : min(sp.few, (keys + 31) / 32);
+  const int ch = attn_head_keys(keys, sp.few);
+  return (keys + ch - 1) / ch;
+}
+__device__ __forceinline__ int attn_keys(const int64_t* __restrict__ pos, int M, int L) {
+  return max(1, (int)min((int64_t)L, pos[M - 1] + 1));
+}
+
+// attention_combine for up to kAttnManyParts partitions, their records room for sp.room: one block per (token, head), a
+// thread per dim; the partitions' weights exp(max - overall max) are evaluated once, a thread each, and shared through LDS
+// (attention_combine has every thread evaluate them all, which its at most 16 partitions hide behind one round trip). Of
+// many tokens the loads of the first 16 partitions go out with the position's, before the partitions' number is known:
+// those that were not written hold anything and are left out (200 tokens on 1000 keys 19.4 -> 17.9 us with the attention;
+// of one token, where most are cold, 12.1 -> 12.9 on 3000). One partition has written out itself.
+__global__ __launch_bounds__(kHeadDim) void attention_combine_many(const float* __restrict__ part,
+                                                                   const int64_t* __restrict__ pos, f16* __restrict__ out,
+                                                                   int M, int Hq, int Hkv, int L, AttnSplit sp) {
   __shared__ float s_max[kAttnManyParts], s_f[kAttnManyParts], s_sum[kAttnManyParts];
   const int m = blockIdx.x / Hq, hd = blockIdx.x % Hq, G = Hq / Hkv, d = threadIdx.x;
-  const float* rec = part + ((size_t)(m * Hkv + hd / G) * P * G + hd % G) * kAttnRec;   // partition p: + p G records
-  const int step = G * kAttnRec;
-  float ps = 0.f;
-  if (d < P) {
-    s_max[d] = rec[(size_t)d * step];
-    ps = rec[(size_t)d * step + 1];
-  }
+  const float* rec = part + ((size_t)(m * Hkv + hd / G) * sp.room * G + hd % G) * kAttnRec;
+  const int step = G * kAttnRec;                            // from one partition's record to the next one's
+  float v[16], pm = -INFINITY, ps = 0.f;
+  auto load_first = [&](int parts) {
+    if (d < parts) {
+      pm = rec[(size_t)d * step];
+      ps = rec[(size_t)d * step + 1];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v[u] = u < parts ? rec[(size_t)u * step + 4 + d] : 0.f;
+  };
+  if (!sp.by_head) load_first(sp.room);
+  const int P = attn_parts(sp, attn_keys(pos, M, L));
+  if (P == 1) return;
+  if (sp.by_head) load_first(P);
+  if (d < P) s_max[d] = pm;
   __syncthreads();
   float gm = -INFINITY;
   for (int p = 0; p < P; ++p) gm = fmaxf(gm, s_max[p]);
   if (d < P) {
-    const float f = s_max[d] == -INFINITY ? 0.f : expf(s_max[d] - gm);   // (a partition that saw no key)
+    const float f = pm == -INFINITY ? 0.f : expf(pm - gm);   // (a partition that saw no key)
     s_f[d] = f;
     s_sum[d] = f * ps;
   }
   __syncthreads();
   float num = 0.f, den = 0.f;
   for (int p0 = 0; p0 < P; p0 += 16) {                       // 16 loads in flight
-    float v[16];
+    if (p0 > 0) {
 #pragma unroll
-    for (int u = 0; u < 16; ++u) v[u] = p0 + u < P ? rec[(size_t)(p0 + u) * step + 4 + d] : 0.f;
+      for (int u = 0; u < 16; ++u) v[u] = p0 + u < P ? rec[(size_t)(p0 + u) * step + 4 + d] : 0.f;
+    }
 #pragma unroll
     for (int u = 0; u < 16; ++u)
       if (p0 + u < P) {
@@ -330,15 +375,14 @@ __global__ __launch_bounds__(kHeadDim) void attention_combine_many(const float* 
 // sum, unnormalized output) of its rows in attention_kernel's layout and attention_combine merges them.
 constexpr int kAttnVtPitch = 80;                            // bytes per dim row of the staged V^T (64 + 16 padding)
 
-__global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, const f16* __restrict__ k_cache,
-                                                     const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
-                                                     f16* __restrict__ out, int M, int Hq, int Hkv, int L, float scale,
-                                                     float* __restrict__ part) {
-  __shared__ __attribute__((aligned(16))) uint8_t vt[kHeadDim * kAttnVtPitch];
-  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, part);
-  const int G = Hq / Hkv, P = gridDim.y, pid = blockIdx.y;
-  const int hk = blockIdx.x % Hkv, tile = blockIdx.x / Hkv;
-  const int lane = threadIdx.x, r = lane & 15, c = lane >> 4;
+// a wave's work: (KV head, row tile) unit, partition pid of P (records of PS), with kHeadDim * kAttnVtPitch bytes of LDS at vt
+__device__ __forceinline__ void attend_mfma(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                            const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
+                                            f16* __restrict__ out, int M, int Hq, int Hkv, int L, float scale,
+                                            float* __restrict__ part, uint8_t* vt, int unit, int pid, int P, int PS) {
+  const int G = Hq / Hkv;
+  const int hk = unit % Hkv, tile = unit / Hkv;
+  const int lane = threadIdx.x & 63, r = lane & 15, c = lane >> 4;
   // this lane's query row (as the B column r)
   const int row = 16 * tile + r, m = row / G, g = row - m * G;
   const bool live = m < M;
@@ -448,13 +492,22 @@ __global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, 
     }
     return;
   }
-  float* mine = part + (((size_t)(m * Hkv + hk) * P + pid) * G + g) * kAttnRec;
+  float* mine = part + (((size_t)(m * Hkv + hk) * PS + pid) * G + g) * kAttnRec;
   if (c == 0) {
     mine[0] = mx;
     mine[1] = lsum;
   }
 #pragma unroll
   for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(mine + 4 + 16 * dt + 4 * c) = o[dt];
+}
+
+__global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                                     const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
+                                                     f16* __restrict__ out, int M, int Hq, int Hkv, int L, float scale,
+                                                     float* __restrict__ part) {
+  __shared__ __attribute__((aligned(16))) uint8_t vt[kHeadDim * kAttnVtPitch];
+  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, part);
+  attend_mfma(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, part, vt, blockIdx.x, blockIdx.y, gridDim.y, gridDim.y);
 }
 
 // Causal GQA attention for prompts and long steps (the contract of attention_mfma): a workgroup of four waves takes
@@ -491,24 +544,23 @@ constexpr float kAttnLagFew = 1.f, kAttnLag = 8.f;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
+// a workgroup's work: bx of tiles * Hkv, partition pid of P (records of PS)
 template <int RG, int KG>
-__global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict__ q, const f16* __restrict__ k_cache,
-                                                           const f16* __restrict__ v_cache,
-                                                           const int64_t* __restrict__ pos, f16* __restrict__ out, int M,
-                                                           int Hq, int Hkv, int L, float scale, int tiles,
-                                                           float* __restrict__ part) {
+__device__ __forceinline__ void attend_prompt(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                              const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
+                                              f16* __restrict__ out, int M, int Hq, int Hkv, int L, float scale, int tiles,
+                                              float* __restrict__ part, uint8_t* smem, int bx, int pid, int P, int PS) {
   static_assert(RG * KG == 4, "four waves");
   constexpr int kRows = 32 * RG, kKeys = 32 * KG;         // query rows of the workgroup, keys of a block
   constexpr int kBuf = kKeys * kHeadDim * 2;                  // bytes of a block's K, and of its V
   constexpr int NP = kKeys / 16;                              // 16-byte pieces a thread loads of K, and of V
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];   // [2][K block, V block]
+  // smem: [2][K block, V block]
   int* s_max = reinterpret_cast<int*>(smem);                  // the waves' last keys, before the first block is staged
-  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, tiles, part);
-  const int G = Hq / Hkv, P = gridDim.y, pid = blockIdx.y;
+  const int G = Hq / Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 31, h = lane >> 5;
   // longest tiles first; every second round of workgroups in reverse, so that a CU's two workgroups add up alike
-  const int hk = blockIdx.x % Hkv, idx = blockIdx.x / Hkv, per = max(1, 256 / Hkv), rnd = idx / per;
+  const int hk = bx % Hkv, idx = bx / Hkv, per = max(1, 256 / Hkv), rnd = idx / per;
   const int at = rnd & 1 ? rnd * per + min(per, tiles - rnd * per) - 1 - (idx - rnd * per) : idx;
   const int tile = tiles - 1 - at;
   const int rgrp = wave % RG, kgrp = wave / RG;               // the wave's rows, and its keys of a block
@@ -703,7 +755,7 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
     return;
   }
   // the record's maximum and sum are natural-base ones: ref / log2(e)
-  float* mine = part + (((size_t)(m * Hkv + hk) * P + pid) * G + g) * kAttnRec;
+  float* mine = part + (((size_t)(m * Hkv + hk) * PS + pid) * G + g) * kAttnRec;
   if (h == 0) {
     mine[0] = ref * 0.69314718055994530942f;
     mine[1] = lsum;
@@ -713,6 +765,57 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
 #pragma unroll
     for (int v = 0; v < 16; v += 4)
       *reinterpret_cast<f32x4*>(mine + 4 + 32 * dt + 2 * v + 4 * h) = f32x4{o[dt][v], o[dt][v + 1], o[dt][v + 2], o[dt][v + 3]};
+}
+
+template <int RG, int KG>
+__global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                                           const f16* __restrict__ v_cache,
+                                                           const int64_t* __restrict__ pos, f16* __restrict__ out, int M,
+                                                           int Hq, int Hkv, int L, float scale, int tiles,
+                                                           float* __restrict__ part) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, tiles, part);
+  attend_prompt<RG, KG>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x, blockIdx.y,
+                        gridDim.y, gridDim.y);
+}
+
+// attend_prompt, or with fewer than sp.from keys attend_heads (HEADS) or attend_mfma, in workgroups of four waves: the work
+// of either is numbered along blockIdx.x, partitions slowest, and workgroups past it end at once. Beside launching one of
+// the kernels by the bound, us on an 8192-row cache with the bound at 8192 (attention_kernel or attention_mfma / attend_prompt
+// alone / this): one token, 16 / 2 heads at position 200 8.7 / 13.6 / 7.3, at 700 11.2 / 13.5 / 8.4, 3000 12.2 / 14.2 /
+// 12.5, 8000 17.2 / 15.0 / 15.4; 28 / 4 heads 10.1 / 13.8 / 7.9, 12.3 / 14.1 / 9.1, 14.9 / 14.7 / 12.2, 28.8 / 16.4 /
+// 16.8; 16 tokens, 16 / 2 heads 8.1 / 13.4 / 7.2, 10.2 / 13.9 / 9.4, 15.8 / 15.1 / 13.7, 29.5 / 17.7 / 17.5. Prompts of
+// 50 .. 200 tokens whose bound is a 4096-row cache: 64 tokens 9.3 / 13.1 / 7.5, on 200 cached 10.7 / 13.3 / 11.5, on 1500
+// 18.6 / 15.1 / 14.7.
+template <int RG, int KG, bool HEADS>
+__global__ __launch_bounds__(256, 2) void attention_select(const f16* __restrict__ q, const f16* __restrict__ k_cache,
+                                                           const f16* __restrict__ v_cache,
+                                                           const int64_t* __restrict__ pos, f16* __restrict__ out, int M,
+                                                           int Hq, int Hkv, int L, float scale, int tiles,
+                                                           float* __restrict__ part, AttnSplit sp) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, tiles, part, sp.from, sp.few, sp.many);
+  const int keys = __builtin_amdgcn_readfirstlane(attn_keys(pos, M, L)), P = attn_parts(sp, keys);
+  if (keys >= sp.from) {
+    const int n = tiles * Hkv, pid = blockIdx.x / n;
+    if (pid < P)
+      attend_prompt<RG, KG>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x - pid * n,
+                            pid, P, sp.room);
+  } else if constexpr (HEADS) {
+    const int n = M * Hq, pid = blockIdx.x / n;
+    const int bx = blockIdx.x - pid * n, G = Hq / Hkv;        // (token, head)
+    if (pid < P)
+      attend_heads<1, 32>(q, k_cache, v_cache, pos, out, Hq, Hkv, L, scale, attn_head_keys(keys, sp.few), part, smem, bx,
+                          pid, P, ((size_t)(bx / G) * sp.room + pid) * G + bx % G);
+  } else {
+    // as many waves a CU as attention_mfma's workgroups of one would put there: two, in one workgroup where no more fit
+    constexpr int NW = KG == 4 ? 2 : 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), unit = NW * blockIdx.x + wave;
+    const int n = (M * (Hq / Hkv) + 15) / 16 * Hkv, pid = unit / n;
+    if (wave < NW && pid < P)
+      attend_mfma(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, part, smem + wave * kHeadDim * kAttnVtPitch,
+                  unit - pid * n, pid, P, sp.room);
+  }
 }
 
 // fp16 GEMV for the (tied) lm_head, M <= 4: y[m][n] = fp16(sum_k x[m][k] W[n][k]), W fp16 [N][K] row-major, fp32
@@ -1104,73 +1207,124 @@ hipError_t launch_attention_mfma(const f16* q, const f16* k, const f16* v, const
   return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
                 Hq);
 }
-// prompts and long caches: one workgroup per (KV head, 32 RG query rows, key partition); partitions while the workgroups
-// number fewer than `target`, at most one per kAttnPromptMinKeys of max_keys, within the workspace (a workgroup splits the
-// keys its rows actually attend, so a bound well above the real count costs only empty partitions)
 template <int RG, int KG>
-hipError_t launch_attention_prompt(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M,
+constexpr size_t prompt_lds() {
+  return std::max<size_t>((size_t)2 * 2 * 32 * KG * kHeadDim * 2, (size_t)(KG - 1) * RG * 66 * 256);
+}
+// key partitions of attend_prompt while its workgroups number fewer than `target`, at most one per kAttnPromptMinKeys of
+// max_keys, within the workspace (a workgroup splits the keys its rows actually attend)
+template <int RG, int KG>
+int prompt_parts(int M, int Hq, int Hkv, int max_keys, const void* ws, size_t ws_bytes, long target) {
+  const long wgs = ((long)M * (Hq / Hkv) + 32 * RG - 1) / (32 * RG) * Hkv;
+  if (!ws || ws_bytes <= kAttnCounterBytes || wgs >= target || max_keys < 2 * kAttnPromptMinKeys) return 1;
+  // (a workgroup of KG = 4 has its CU to itself: one round of them)
+  const long P = std::min<long>({KG == 4 ? std::max(1L, 256 / wgs) : (target + wgs - 1) / wgs, (max_keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys,
+                                 (long)kAttnManyParts});
+  const size_t per = (size_t)M * Hq * kAttnRec * sizeof(float);
+  return (int)std::max<size_t>(1, std::min<size_t>((size_t)P, (ws_bytes - kAttnCounterBytes) / per));
+}
+float* attn_partials(void* ws) {
+  return ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kAttnCounterBytes) : nullptr;
+}
+// prompts whose keys number few: one workgroup per (KV head, 64 query rows, key partition)
+hipError_t launch_attention_prompt(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
+                                   int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
+  const int G = Hq / Hkv;
+  const int tiles = (int)(((long)M * G + 63) / 64);
+  const int P = max_keys < kAttnPromptSplitKeys ? 1 : prompt_parts<2, 2>(M, Hq, Hkv, max_keys, ws, ws_bytes, 512);
+  static_assert(prompt_lds<2, 2>() <= 65536 && kAttnPromptLongKeys / kAttnPromptMinKeys <= kAttnMaxParts, "");
+  hipError_t e = launch(attention_prompt<2, 2>, dim3((unsigned)(tiles * Hkv), P), dim3(256), prompt_lds<2, 2>(), st, q, k, v,
+                        pos, out, M, Hq, Hkv, L, scale, tiles, attn_partials(ws));
+  if (e != hipSuccess || P == 1) return e;
+  const long threads = (long)M * Hq * kHeadDim;
+  return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, attn_partials(ws), out, M * Hkv,
+                G, P, Hq);
+}
+// attention_select: the launch holds both kernels' workgroups
+template <int RG, int KG, bool HEADS>
+hipError_t launch_attention_select(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M,
                                    int Hq, int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes,
-                                   hipStream_t st, long target) {
+                                   hipStream_t st, long target, int from) {
   const int G = Hq / Hkv;
   const int tiles = (int)(((long)M * G + 32 * RG - 1) / (32 * RG));
-  const long wgs = (long)tiles * Hkv;
-  int P = 1;
-  if (ws && ws_bytes > kAttnCounterBytes && wgs < target && max_keys >= 2 * kAttnPromptMinKeys) {
-    P = (int)std::min<long>({(target + wgs - 1) / wgs, (max_keys + kAttnPromptMinKeys - 1) / kAttnPromptMinKeys,
-                             (long)kAttnManyParts});
+  AttnSplit sp{from, 1, prompt_parts<RG, KG>(M, Hq, Hkv, max_keys, ws, ws_bytes, target), HEADS, 1};
+  const long units = HEADS ? (long)M * Hq : ((long)M * G + 15) / 16 * Hkv, room = HEADS ? kAttnSelectBlocks : kAttnMfmaTargetWaves;
+  const int few_keys = std::min(max_keys, from - 1), least = HEADS ? 128 : kAttnMinKeys;
+  if (ws && ws_bytes > kAttnCounterBytes && units < room && few_keys >= 2 * least) {
     const size_t per = (size_t)M * Hq * kAttnRec * sizeof(float);
-    P = (int)std::max<size_t>(1, std::min<size_t>((size_t)P, (ws_bytes - kAttnCounterBytes) / per));
+    sp.few = (int)std::min<long>({(room + units - 1) / units, (few_keys + least - 1) / least,
+                                  (long)(HEADS ? kAttnManyParts : kAttnMaxParts), (long)((ws_bytes - kAttnCounterBytes) / per)});
+    sp.few = std::max(sp.few, 1);
   }
-  float* part = ws ? reinterpret_cast<float*>(static_cast<uint8_t*>(ws) + kAttnCounterBytes) : nullptr;
-  constexpr size_t lds = std::max<size_t>((size_t)2 * 2 * 32 * KG * kHeadDim * 2, (size_t)(KG - 1) * RG * 66 * 256);
+  sp.room = std::max(sp.few, sp.many);
+  constexpr size_t lds = prompt_lds<RG, KG>();
+  static_assert(lds >= (size_t)2 * kHeadDim * kAttnVtPitch, "attend_mfma's V");
+  const long few_blocks = HEADS || KG != 4 ? units * sp.few : (units * sp.few + 1) / 2;
   if (lds > 65536) {
-    static const hipError_t attr = allow_lds(attention_prompt<RG, KG>, lds);
+    static const hipError_t attr = allow_lds(attention_select<RG, KG, HEADS>, lds);
     if (attr != hipSuccess) return attr;
   }
-  hipError_t e = launch(attention_prompt<RG, KG>, dim3((unsigned)wgs, P), dim3(256), lds, st, q, k, v, pos, out, M, Hq, Hkv,
-                        L, scale, tiles, part);
-  if (e != hipSuccess || P == 1) return e;
-  if (P > kAttnMaxParts)
-    return launch(attention_combine_many, dim3((unsigned)(M * Hq)), dim3(kHeadDim), 0, st, part, out, Hq, Hkv, P);
-  const long threads = (long)M * Hq * kHeadDim;
-  return launch(attention_combine, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, part, out, M * Hkv, G, P,
-                Hq);
+  hipError_t e = launch(attention_select<RG, KG, HEADS>, dim3((unsigned)std::max((long)tiles * Hkv * sp.many, few_blocks)),
+                        dim3(256), lds, st, q, k, v, pos, out, M, Hq, Hkv, L, scale, tiles, attn_partials(ws), sp);
+  if (e != hipSuccess || sp.room == 1) return e;
+  return launch(attention_combine_many, dim3((unsigned)(M * Hq)), dim3(kHeadDim), 0, st, attn_partials(ws), pos, out, M, Hq,
+                Hkv, L, sp);
 }
-// Long caches: few query rows over many keys go to the prompt kernel with the keys split over the chip, where the decode
-// kernel has every query head read K and V on its own (Hq / Hkv times) and attention_mfma's waves load theirs unshared,
-// both at most 16 ways. Its longer prologue and the merge of up to 64 partitions cost ~11 us at any length, so it starts
-// where the others pass that: 2048 keys, and M Hq keys from 80 K (one token: 128 K, since the others can leave the merge to
-// the o projection). MI355X, us (others -> this): one token, 28 / 4 heads, 3000 keys 16.7 -> 12.1, 16000 45 -> 19, 24000 64 -> 21
-// (12 / 2 heads 6000 13.3 -> 13.9, 12000 18.3 -> 16.5, 24000 28 -> 19); 4 tokens of 16 / 2 heads on 6000 23.4 -> 14.7;
-// 16 on 3000 16.1 -> 14.1 (1500: 11.2 against 11.9), 24000 72 -> 24. `max_keys` is the caller's bound; the partitions
-// follow the real count. A workspace of fewer than 16 partitions keeps the other kernels.
-bool long_attention(int M, int Hq, int Hkv, int max_keys, size_t ws_bytes) {
-  const long rows = (long)M * (Hq / Hkv);
-  if (rows >= kAttnPromptMinRows || max_keys < kAttnLongKeys) return false;
-  if ((long)M * Hq * max_keys < (M == 1 ? kAttnLongWorkOne : kAttnLongWork)) return false;
-  return ws_bytes >= kAttnCounterBytes + (size_t)16 * M * Hq * kAttnRec * sizeof(float);
+// Which kernel serves a call. attend_prompt shares K and V among a KV head's rows and splits the keys over the chip up to
+// kAttnManyParts ways, where attention_kernel has every query head read them on its own and attention_mfma's waves load
+// theirs unshared, both at most 16 ways; its prologue and merge cost more. Its figures here are with a bound equal to the
+// keys (others -> it).
+//   Few rows (below kAttnPromptMinRows per KV head) from 2048 keys and M Hq keys of 80 K, one token from 128 K (the others
+//   can leave its merge to the o projection): us, one token, 28 / 4 heads, 3000 keys 16.7 -> 12.1, 16000 45 -> 19, 24000
+//   65 -> 22; 12 / 2 heads 12000 18.3 -> 16.5; 4 tokens of 16 / 2 heads on 6000 23.4 -> 14.7; 16 on 3000 16.1 -> 14.1
+//   (1500: 11.2 against 11.9). With one query head per KV head there is nothing to share below 16 rows (one token, 16 / 16
+//   heads on 16000 keys 29.9 -> 32.9; 2 heads per KV head 26.2 -> 22.9), and steps of 64 or more (token, KV head)s below 32
+//   rows keep attention_kernel. A workspace of fewer than 16 partitions keeps the others, too: that of 4 MB which the
+//   Python binding gives serves M Hq <= 496.
+//   More rows from M Hq keys of 560 K: 16 / 2 heads, 48 tokens on 256 cached 9.5 -> 11.5, on 512 11.0 -> 11.9, on 1500 16.4
+//   -> 14.8; 64 tokens 5.5 -> 7.7, on 256 cached 10.3 -> 11.8, on 512 12.2 level, on 1000 15.8 -> 14.6; 128 tokens, which
+//   stay below it, 10.6 -> 8.6, on 128 13.0 -> 10.7, on 512 18.1 -> 15.1.
+// attn_bound_from: the keys from which a call's bound on them lets attend_prompt serve it (0: never). attn_keys_from: those
+// from which, in attention_select, it then does (one token 50 K Hq keys, few rows 76 K M Hq keys, up to 383 rows 2048 keys,
+// beyond 192: where the two bodies crossed in sweeps of 200 .. 16000 keys on 4096- to 16384-row caches).
+int attn_bound_from(int M, int Hq, int Hkv, size_t ws_bytes) {
+  const int G = Hq / Hkv;
+  const long rows = (long)M * G, work = (long)M * Hq;
+  if (rows >= kAttnPromptMinRows) return (int)std::max<long>(1, (kAttnPromptWork + work - 1) / work);
+  if (G == 1 && rows < 16) return 0;
+  if (rows < kAttnMfmaMinRows && (long)M * Hkv >= 64) return 0;
+  if (ws_bytes < kAttnCounterBytes + (size_t)16 * M * Hq * kAttnRec * sizeof(float)) return 0;
+  return (int)std::max<long>(kAttnLongKeys, ((M == 1 ? kAttnLongWorkOne : kAttnLongWork) + work - 1) / work);
 }
-hipError_t launch_attention_long(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
-                                 int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
-  // 64 rows a workgroup up to 128 rows, 32 beyond (28 / 4 heads, 32 tokens on 24000: 43 us against 53; 16 / 2, 16 on 24000:
-  // 24 against 27)
-  if ((long)M * (Hq / Hkv) <= 128)
-    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256);
-  return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256);
+int attn_keys_from(int M, int Hq, int Hkv) {
+  const long rows = (long)M * (Hq / Hkv), work = (long)M * Hq;
+  if (rows >= kAttnPromptMinRows) return kAttnPromptKeysFrom;
+  if (rows >= kAttnMfmaMinRows) return kAttnRowsKeysFrom;
+  return (int)(((M == 1 ? kAttnOneWorkFrom : kAttnFewWorkFrom) + work - 1) / work);
 }
 }  // namespace
 
 hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int64_t* pos, f16* out, int M, int Hq,
                             int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
   const long rows = (long)M * (Hq / Hkv);
-  // the prompt kernel's longer prologue and merge pay from about 384 rows (16 / 2 heads, 48 tokens on 600 cached: level
-  // at 12.9 us; 28 / 4 heads, 64 on 1000: 21.7 -> 17.1; below: 16 tokens on 512 cached 9.0 against 11.4 us)
-  if (long_attention(M, Hq, Hkv, max_keys, ws ? ws_bytes : 0))
-    return launch_attention_long(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
-  if (rows >= kAttnPromptMinRows) {
-    if ((rows + 63) / 64 * Hkv < kAttnPromptWide && max_keys >= kAttnPromptLongKeys)
-      return launch_attention_prompt<1, 4>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512);
-    return launch_attention_prompt<2, 2>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512);
+  if (!ws) ws_bytes = 0;
+  const int bound_from = attn_bound_from(M, Hq, Hkv, ws_bytes);
+  int from = attn_keys_from(M, Hq, Hkv);
+  if (bound_from > 0 && max_keys >= bound_from) {
+    if (rows < kAttnMfmaMinRows)
+      return launch_attention_select<2, 2, true>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
+    // 64 rows a workgroup up to 128 rows, 32 beyond (28 / 4 heads, 32 tokens on 24000: 43 us against 53; 16 / 2, 16 on
+    // 24000: 24 against 27)
+    if (rows <= 128)
+      return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
+    if (rows < kAttnPromptMinRows)
+      return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
+    if (max_keys < kAttnPromptLongKeys)
+      return launch_attention_prompt(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+    if (M >= from) from = 1;                                  // (M tokens attend M keys at least, unless they share positions)
+    if ((rows + 63) / 64 * Hkv < kAttnPromptWide)
+      return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, from);
+    return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, from);
   }
   if (rows >= kAttnMfmaMinRows)
     return launch_attention_mfma(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
@@ -1192,12 +1346,14 @@ hipError_t attention_partials_launch(const f16* q, const f16* k, const f16* v, c
                                      hipStream_t st) {
   // one token: the decode kernel with one query head per block (the MFMA kernel takes 32 or more rows per KV head)
   if (Hq / Hkv >= kAttnMfmaMinRows || Hkv >= 64) return hipErrorInvalidValue;
-  // a long cache: merged here, into out; the partials then start behind out in the workspace (out [Hq * 128] is its start)
+  // a bound of a long cache: merged here, into out, as attention_launch does; the partials then follow out in the workspace
   const size_t xbytes = (size_t)Hq * kHeadDim * sizeof(f16);
-  if (ws_bytes > xbytes && long_attention(1, Hq, Hkv, max_keys, ws_bytes - xbytes)) {
+  const int bound_from = ws_bytes > xbytes ? attn_bound_from(1, Hq, Hkv, ws_bytes - xbytes) : 0;
+  if (bound_from > 0 && max_keys >= bound_from) {
     *parts = 1;
-    return launch_attention_long(q, k, v, pos, out, 1, Hq, Hkv, L, max_keys, scale, static_cast<uint8_t*>(ws) + xbytes,
-                                 ws_bytes - xbytes, st);
+    return launch_attention_select<2, 2, true>(q, k, v, pos, out, 1, Hq, Hkv, L, max_keys, scale,
+                                               static_cast<uint8_t*>(ws) + xbytes, ws_bytes - xbytes, st, 256,
+                                               attn_keys_from(1, Hq, Hkv));
   }
   return launch_attention<1, 32>(q, k, v, pos, out, 1, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, kAttnXMaxParts,
                                  false, parts);

@@ -283,16 +283,25 @@ constexpr size_t kAttnCounterBytes = 4096;
 // splits keys while its waves number fewer than kAttnMfmaTargetWaves
 constexpr int kAttnMfmaMinRows = 32;
 constexpr int kAttnMfmaTargetWaves = 512;
-// the prompt attention takes steps with at least kAttnPromptMinRows query rows per KV head, with 64 rows a workgroup, or
-// 32 where those leave CUs idle (fewer than kAttnPromptWide workgroups) and there are keys to share out
+// the prompt attention (decode_ops.hip, attn_bound_from): steps of kAttnPromptMinRows or more query rows per KV head from
+// kAttnPromptWork (token, head, key)s, of fewer from kAttnLongKeys keys and kAttnLongWork(One); with 64 rows a workgroup, or
+// 32 where those leave CUs idle (fewer than kAttnPromptWide workgroups) and a bound of kAttnPromptLongKeys keys or more
 constexpr int kAttnPromptMinRows = 384;
+constexpr long kAttnPromptWork = 560000;
 constexpr int kAttnPromptWide = 160;
 constexpr int kAttnPromptLongKeys = 1024;
-constexpr int kAttnManyParts = 64;        // its key partitions at most
-// fewer rows go there too from kAttnLongKeys keys and this many (token, head, key)s
 constexpr int kAttnLongKeys = 2048;
 constexpr long kAttnLongWork = 80000, kAttnLongWorkOne = 128000;
+// its key partitions: at most kAttnManyParts, of at least kAttnPromptMinKeys keys; a bound below kAttnPromptSplitKeys leaves
+// the keys whole, without the merge's launch (16 / 2 heads, 192 tokens on 64 cached 15.0 -> 10.1 us)
+constexpr int kAttnManyParts = 64;
 constexpr int kAttnPromptMinKeys = 128;
+constexpr int kAttnPromptSplitKeys = 384;
+// under a bound that may lie above the keys (attn_keys_from, attention_select): workgroups that one-token and few-row steps
+// spread over, and the keys from which the prompt attention takes over
+constexpr int kAttnSelectBlocks = 1024;
+constexpr int kAttnPromptKeysFrom = 192, kAttnRowsKeysFrom = 2048;
+constexpr long kAttnOneWorkFrom = 50000, kAttnFewWorkFrom = 76000;
 constexpr int kAttnManyBlocks = 512;      // from this many blocks on, at most 4 waves per block
 constexpr int kMaxSplits = 32;
 constexpr size_t kCounterBytes = 16384;

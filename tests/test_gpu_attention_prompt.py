@@ -136,3 +136,82 @@ def test_long_tail_of_small_weights(cuda, m, drop, floor):
     assert bool((want > 1e-4).all())
     err = (out.double() - want).norm() / want.norm()
     assert err < BOUND + 2.0 ** (drop - floor), float(err)
+
+
+# bounds far above the keys: the kernel is chosen on the device by the last token's position, one token, few rows (attend_heads
+# below), up to 128 and 383 rows and prompts (attend_mfma below), keys on either side of each line and at partition edges;
+# the last column sends the last token's position below the others'
+@pytest.mark.parametrize("m,hq,hkv,L,keys", [
+    (1, 16, 2, 8192, (1, 2, 127, 128, 129, 2049, 3124, 3125, 3126, 8192)), (1, 28, 4, 4608, (33, 1785, 1786, 1787, 4608)),
+    (1, 16, 8, 16384, (64, 3125, 9000)), (3, 28, 4, 2048, (3, 500, 904, 905, 2048)), (2, 12, 2, 4096, (2, 3166, 3167, 4000)),
+    (4, 16, 2, 4096, (4, 64, 65, 2047, 2048, 4096)), (16, 16, 2, 4096, (16, 31, 700, 2048, 3000)),
+    (17, 16, 2, 2560, (17, 65, 600, 2047, 2048, 2560)), (16, 16, 16, 4096, (16, 3000)), (30, 12, 2, 4096, (40, 700, 3000)),
+    (48, 16, 2, 4096, (48, 64, 65, 191, 192, 1500)), (55, 28, 4, 1200, (55, 192, 567, 1200)), (96, 12, 2, 2048, (96, 191, 400)),
+    (200, 16, 2, 2048, (200, 300, 2048)), (400, 4, 4, 1664, (400, 1600)), (8, 8, 8, 8192, (8, 5000))])
+def test_bound_above_the_keys(cuda, m, hq, hkv, L, keys):
+    q, k, v = case(m, hq, hkv, L, m + L)
+    clean = k, v
+    for n in keys:
+        k, v = clean[0].clone(), clean[1].clone()
+        k[:, n:] = float("nan")
+        v[:, n:] = float("nan")
+        pos = torch.arange(n - m, n, device="cuda") if n >= m else torch.full((m,), n - 1, device="cuda")
+        one = check(q, k, v, pos, 128 ** -0.5, n)
+        assert torch.equal(one, check(q, k, v, pos, 128 ** -0.5, n))
+        check(q, k, v, pos.flip(0).contiguous(), 128 ** -0.5, n)
+        if n >= m:
+            last_low = pos.clone()
+            last_low[-1] = 0
+            check(q, k, v, last_low, 128 ** -0.5, n)
+
+
+@pytest.mark.parametrize("m,hq,hkv,L", [(1, 16, 2, 8192), (3, 28, 4, 4096), (16, 16, 2, 8192), (24, 16, 2, 2560),
+                                        (64, 16, 2, 4096)])
+def test_captured_once_for_every_position(cuda, m, hq, hkv, L):
+    """A graph captured at one position serves the others: every replay has the eager call's bits, on both sides of the
+    line and back, with eager calls between the replays."""
+    q, k, v = case(m, hq, hkv, L, 3 * m)
+    pos = torch.arange(m, device="cuda")
+    out = torch.empty(m, hq * 128, dtype=torch.float16, device="cuda")
+    call = lambda o: ops.ext().attention(q, k, v, pos, o, hq, hkv, L, 128 ** -0.5)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call(out)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=side):
+        call(out)
+    for first in (0, 100, L - m, 30, 1000, 2500 if L > 2600 else 1500, 7):
+        pos.copy_(torch.arange(first, first + m, device="cuda"))
+        eager = torch.empty_like(out)
+        call(eager)
+        out.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), first
+        check(q, k, v, pos, 128 ** -0.5, first + m)
+
+
+@pytest.mark.parametrize("m,hq,hkv,L,last", [(47, 16, 2, 2048, 2000), (54, 28, 4, 2304, 2176), (18, 28, 4, 2560, 2500),
+                                             (47, 16, 2, 2048, 60)])
+def test_long_cache_attention_in_a_workspace_of_its_size(cuda, m, hq, hkv, L, last):
+    """Steps whose 16 partitions the Python binding's workspace does not hold, through the C ABI: with a workspace that
+    holds them exactly and one that falls 16 bytes short (the other kernel), and nothing written past either."""
+    from lowbit import _native
+    q, k, v = case(m, hq, hkv, L, m)
+    k[:, last + 1:] = float("nan")
+    v[:, last + 1:] = float("nan")
+    pos = torch.arange(last + 1 - m, last + 1, device="cuda")
+    want = attend(q, k[:, :last + 1], v[:, :last + 1], pos, 128 ** -0.5).view(m, -1)
+    need = 4096 + 16 * m * hq * 132 * 4
+    for size in (need, need - 16, 2 * need):
+        ws = torch.full((size + 4096,), 171, dtype=torch.uint8, device="cuda")
+        out = torch.empty(m, hq * 128, dtype=torch.float16, device="cuda")
+        _native.check(_native.lib().lowbit_attention(
+            _native.ptr(q), _native.ptr(k), _native.ptr(v), _native.ptr(pos), _native.ptr(out), m, hq, hkv, L, L, 128 ** -0.5,
+            _native.ptr(ws), size, torch.cuda.current_stream().cuda_stream))
+        err = (out.double() - want).norm() / want.norm()
+        assert err < BOUND, (size, float(err))
+        assert bool((ws[size:] == 171).all()) and bool((ws[:4096] == 171).all())
