@@ -184,6 +184,12 @@ int lowbit_w4_gemm_prefill(const void* x, const void* w, const void* s, void* y,
                            int64_t group, int epilogue, const void* aux, void* workspace, size_t workspace_bytes,
                            void* stream);
 
+/* The launch that lowbit_w4_gemm_prefill makes for x [M, K], N weight rows and a workspace of workspace_bytes (0: none),
+ * under the tuning override, for tests and tuning sweeps (host only): plan[0] activation rows and plan[1] weight rows of a
+ * tile, plan[2] the workgroups that split K of a split tile, plan[3] the tiles that one workgroup each takes whole, plan[4]
+ * the workgroups of the launch. */
+int lowbit_w4_prefill_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int* plan);
+
 /* out[M][H] = weight * fp16(x / sqrt(mean(x^2) + eps)) (fp16 in/out, fp32 statistics; transformers Qwen2RMSNorm). */
 int lowbit_rmsnorm(const void* x, const void* weight, void* out, int64_t M, int64_t H, float eps, void* stream);
 

@@ -1,6 +1,7 @@
 // The C ABI (include/lowbit_w4.h): argument validation with the reference's messages, then dispatch to the kernels.
 // The validation mirrors the reference's check() / TORCH_CHECKs (csrc/w4_gemv.cu:312-325,454-540); checks that need
 // tensor metadata (device, dtype, contiguity, dims) are done by the Python layer, which owns the tensors.
+#include <algorithm>
 #include <atomic>
 #include <climits>
 #include <cstring>
@@ -357,6 +358,17 @@ int lowbit_w4_gemm_prefill(const void* x, const void* w, const void* s, void* y,
   a.epi.mode = epilogue;
   a.epi.aux = static_cast<const f16*>(aux);
   return hip_status(gemm_prefill_launch(a, workspace, workspace_bytes), "w4_gemm_prefill");
+}
+
+int lowbit_w4_prefill_plan(int64_t M, int64_t N, int64_t K, size_t workspace_bytes, int* plan) {
+  if (!plan) return fail(LOWBIT_ERR_ARG, "null pointer argument");
+  if (M < 1) return fail(LOWBIT_ERR_ROWS, "the prefill GEMM takes at least one row");
+  if (N < 1 || !fits_int(N) || K < 128 || K > kMaxK || (M + 128) * K * 2 > INT_MAX) return fail(LOWBIT_ERR_SHAPE, "shape mismatch");
+  if (K % 128) return fail(LOWBIT_ERR_LAYOUT, "the MFMA layout needs K to be a multiple of 128");
+  const PrefillPlan p = plan_gemm_prefill((int)M, (int)N, (int)K, workspace_bytes);
+  const int v[5] = {16 * p.MT, 64 * p.PT, p.S, p.full, p.items};
+  std::copy(v, v + 5, plan);
+  return ok();
 }
 
 int lowbit_rmsnorm(const void* x, const void* weight, void* out, int64_t M, int64_t H, float eps, void* stream) {

@@ -43,6 +43,7 @@ SIGNATURES = {
                                 ctypes.c_size_t, _vp], _int),
     "lowbit_w4_gemm_prefill": ([_vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp, _vp, ctypes.c_size_t, _vp],
                                _int),
+    "lowbit_w4_prefill_plan": ([_i64, _i64, _i64, ctypes.c_size_t, ctypes.POINTER(_int)], _int),
     "lowbit_rmsnorm": ([_vp, _vp, _vp, _i64, _i64, ctypes.c_float, _vp], _int),
     "lowbit_rope_kv": ([_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp], _int),
     "lowbit_w4_qkv_rope": ([_vp, _vp, _vp, _i64, _i64, _i64, _vp, _vp, ctypes.c_float, _vp, _vp, _vp, _vp, _vp, _i64,

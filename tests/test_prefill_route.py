@@ -140,3 +140,28 @@ def test_results_are_plain_tensors(monkeypatch):
     for v in (x, x.as_subclass(Sub), torch.nn.Parameter(x)):
         y = _native._output_rows(v, 3, 5)
         assert type(y) is torch.Tensor and y.shape == (3, 5) and y.dtype is torch.float16 and not y.requires_grad
+
+
+@pytest.mark.parametrize("workspace", [0, 16384, 16384 + (1 << 20), 16384 + (64 << 20)])
+def test_prefill_plans_fit(workspace):
+    """The launch shape of the prefill GEMM over its range (host only): every tile is covered once, whole or in splits of
+    at least four chunks, with an arrival counter a split tile and partials within the workspace; whole tiles before split
+    ones fill whole rounds, so that the workgroup numbering of both starts on a multiple of the eight XCDs."""
+    import ctypes
+    p = (ctypes.c_int * 5)()
+    shapes = set()
+    for k in (128, 384, 896, 2048, 3584, 11008, 18944):
+        for n in (1, 64, 250, 1536, 2048, 2560, 4604, 11008, 18944, 22016):
+            for m in (1, 64, 65, 100, 200, 333, 512, 700, 1000, 1400, 2048, 5000):
+                _native.check(_native.lib().lowbit_w4_prefill_plan(m, n, k, workspace, p))
+                rows, cols, split, whole, groups = p
+                shapes.add((rows, cols, split > 1, whole > 0))
+                tiles = -(-m // rows) * -(-n // cols)
+                rest = tiles - whole
+                assert groups == whole + split * rest and whole >= 0 and rest >= 0
+                assert rest == 0 or split > 1 and k // 128 >= 4 * split and rest <= 4096
+                assert rest == 0 or whole % 256 == 0
+                assert rest == 0 or 16384 + rest * split * rows * cols * 4 <= workspace
+    assert {s[:2] for s in shapes} == {(64, 64), (64, 128), (96, 256), (128, 128)}
+    if workspace > 1 << 25:
+        assert {s[:2] for s in shapes if s[2] and s[3]} >= {(96, 256), (128, 128)}
