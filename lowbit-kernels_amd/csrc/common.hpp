@@ -2,6 +2,8 @@
 // reductions (DPP + readlane, no LDS), buffer-resource loads and the launch helper.
 #pragma once
 #include <hip/hip_runtime.h>
+
+#include <atomic>
 #include <cstdint>
 
 namespace lowbit {
@@ -342,6 +344,18 @@ template <typename... KArgs>
 inline hipError_t allow_lds(void (*kernel)(KArgs...), size_t bytes) {
   return hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
                              (int)bytes);
+}
+
+// The same once for each GPU of the process (the limit is the loaded function's, one a GPU); `done` is the kernel's own.
+template <typename... KArgs>
+inline hipError_t allow_lds_once(std::atomic<uint64_t>& done, void (*kernel)(KArgs...), size_t bytes) {
+  int dev = 0;
+  if (hipError_t e = hipGetDevice(&dev)) return e;
+  const uint64_t bit = dev < 64 ? (uint64_t)1 << dev : 0;
+  if (done.load(std::memory_order_relaxed) & bit) return hipSuccess;
+  if (hipError_t e = allow_lds(kernel, bytes)) return e;
+  done.fetch_or(bit, std::memory_order_relaxed);
+  return hipSuccess;
 }
 
 }  // namespace lowbit

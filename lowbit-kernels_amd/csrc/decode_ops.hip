@@ -1064,8 +1064,8 @@ template <int MT, int D>
 hipError_t launch_f16w_rows(const f16* x, const f16* w, f16* y, int M, int N, int K, hipStream_t st) {
   constexpr size_t lds = (size_t)D * (4 + MT) * 16 * 256;
   if (lds > 65536) {
-    static const hipError_t attr = allow_lds(gemm_f16w_rows_kernel<MT, D>, lds);
-    if (attr != hipSuccess) return attr;
+    static std::atomic<uint64_t> done{0};
+    if (hipError_t e = allow_lds_once(done, gemm_f16w_rows_kernel<MT, D>, lds)) return e;
   }
   return launch(gemm_f16w_rows_kernel<MT, D>, dim3((unsigned)((N + 63) / 64)), dim3(256), lds, st, x, w, y, M, N, K);
 }
@@ -1261,8 +1261,8 @@ hipError_t launch_attention_select(const f16* q, const f16* k, const f16* v, con
   static_assert(lds >= (size_t)2 * kHeadDim * kAttnVtPitch, "attend_mfma's V");
   const long few_blocks = HEADS || KG != 4 ? units * sp.few : (units * sp.few + 1) / 2;
   if (lds > 65536) {
-    static const hipError_t attr = allow_lds(attention_select<RG, KG, HEADS>, lds);
-    if (attr != hipSuccess) return attr;
+    static std::atomic<uint64_t> done{0};
+    if (hipError_t e = allow_lds_once(done, attention_select<RG, KG, HEADS>, lds)) return e;
   }
   hipError_t e = launch(attention_select<RG, KG, HEADS>, dim3((unsigned)std::max((long)tiles * Hkv * sp.many, few_blocks)),
                         dim3(256), lds, st, q, k, v, pos, out, M, Hq, Hkv, L, scale, tiles, attn_partials(ws), sp);
