@@ -544,12 +544,13 @@ constexpr float kAttnLagFew = 1.f, kAttnLag = 8.f;
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
-// a workgroup's work: bx of tiles * Hkv, partition pid of P (records of PS)
-template <int RG, int KG>
+// a workgroup's work: bx of tiles * Hkv, partition pid of P (records of PS); FEW: below kAttnMfmaMinRows rows; one: the last
+// key of a one-token call, where the caller has read it, else -1
+template <int RG, int KG, bool FEW>
 __device__ __forceinline__ void attend_prompt(const f16* __restrict__ q, const f16* __restrict__ k_cache,
                                               const f16* __restrict__ v_cache, const int64_t* __restrict__ pos,
                                               f16* __restrict__ out, int M, int Hq, int Hkv, int L, float scale, int tiles,
-                                              float* __restrict__ part, uint8_t* smem, int bx, int pid, int P, int PS) {
+                                              float* __restrict__ part, uint8_t* smem, int bx, int pid, int P, int PS, int one) {
   static_assert(RG * KG == 4, "four waves");
   constexpr int kRows = 32 * RG, kKeys = 32 * KG;         // query rows of the workgroup, keys of a block
   constexpr int kBuf = kKeys * kHeadDim * 2;                  // bytes of a block's K, and of its V
@@ -566,19 +567,28 @@ __device__ __forceinline__ void attend_prompt(const f16* __restrict__ q, const f
   const int rgrp = wave % RG, kgrp = wave / RG;               // the wave's rows, and its keys of a block
   const int row = kRows * tile + 32 * rgrp + j, m = row / G, g = row - m * G;
   const bool live = m < M;
-  const int pr = live ? (int)min((int64_t)L - 1, pos[m]) : -1;    // last key the row attends
-  int wmax = pr, wmin = live ? pr : INT_MAX;                  // the wave's last key, and its rows' first last key
+  int pr, wmax, wmin, gmax;                                   // the last keys: the row's, the wave's largest and least, all
+  if (one >= 0) {                                             // one token, whose position the caller has read
+    pr = live ? one : -1;
+    wmax = rgrp == 0 ? one : -1;
+    wmin = rgrp == 0 ? one : INT_MAX;
+    gmax = one;
+  } else {
+    pr = live ? (int)min((int64_t)L - 1, pos[m]) : -1;
+    wmax = pr;
+    wmin = live ? pr : INT_MAX;
 #pragma unroll
-  for (int o = 1; o < 32; o <<= 1) {
-    wmax = max(wmax, __shfl_xor(wmax, o, 64));
-    wmin = min(wmin, __shfl_xor(wmin, o, 64));
+    for (int o = 1; o < 32; o <<= 1) {
+      wmax = max(wmax, __shfl_xor(wmax, o, 64));
+      wmin = min(wmin, __shfl_xor(wmin, o, 64));
+    }
+    wmax = __builtin_amdgcn_readfirstlane(wmax);
+    wmin = __builtin_amdgcn_readfirstlane(wmin);
+    if (lane == 0) s_max[wave] = wmax;
+    __syncthreads();
+    gmax = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
+    __syncthreads();
   }
-  wmax = __builtin_amdgcn_readfirstlane(wmax);
-  wmin = __builtin_amdgcn_readfirstlane(wmin);
-  if (lane == 0) s_max[wave] = wmax;
-  __syncthreads();
-  const int gmax = max(max(s_max[0], s_max[1]), max(s_max[2], s_max[3]));
-  __syncthreads();
   const int ch = ((gmax + 1 + P - 1) / P + kKeys - 1) / kKeys * kKeys;
   const int kbeg = pid * ch, kend = min(gmax + 1, kbeg + ch);
   // q of row j, dims 16 ks + 8 h .. + 7; a negative scale is moved into q (exact), so that score order is weight order
@@ -624,7 +634,7 @@ __device__ __forceinline__ void attend_prompt(const f16* __restrict__ q, const f
     const s16x4 c = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(smem + at + 2048));
     return __builtin_bit_cast(f16x8, __builtin_shufflevector(a, c, 0, 1, 2, 3, 4, 5, 6, 7));
   };
-  const float lag = M * G < kAttnMfmaMinRows ? kAttnLagFew : kAttnLag;
+  constexpr float lag = FEW ? kAttnLagFew : kAttnLag;
   float ref = -INFINITY, lsum = 0.f;                          // reference (base 2), the lane's share of the weights' sum
   f32x16 o[4];
 #pragma unroll
@@ -775,8 +785,8 @@ __global__ __launch_bounds__(256, 2) void attention_prompt(const f16* __restrict
                                                            float* __restrict__ part) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   args_in_sgprs(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, tiles, part);
-  attend_prompt<RG, KG>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x, blockIdx.y,
-                        gridDim.y, gridDim.y);
+  attend_prompt<RG, KG, false>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x, blockIdx.y,
+                        gridDim.y, gridDim.y, -1);
 }
 
 // attend_prompt, or with fewer than sp.from keys attend_heads (HEADS) or attend_mfma, in workgroups of four waves: the work
@@ -799,8 +809,8 @@ __global__ __launch_bounds__(256, 2) void attention_select(const f16* __restrict
   if (keys >= sp.from) {
     const int n = tiles * Hkv, pid = blockIdx.x / n;
     if (pid < P)
-      attend_prompt<RG, KG>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x - pid * n,
-                            pid, P, sp.room);
+      attend_prompt<RG, KG, HEADS>(q, k_cache, v_cache, pos, out, M, Hq, Hkv, L, scale, tiles, part, smem, blockIdx.x - pid * n,
+                            pid, P, sp.room, HEADS && M == 1 ? keys - 1 : -1);
   } else if constexpr (HEADS) {
     const int n = M * Hq, pid = blockIdx.x / n;
     const int bx = blockIdx.x - pid * n, G = Hq / Hkv;        // (token, head)
@@ -1281,16 +1291,24 @@ hipError_t launch_attention_select(const f16* q, const f16* k, const f16* v, con
 //   heads on 16000 keys 29.9 -> 32.9; 2 heads per KV head 26.2 -> 22.9), and steps of 64 or more (token, KV head)s below 32
 //   rows keep attention_kernel. A workspace of fewer than 16 partitions keeps the others, too: that of 4 MB which the
 //   Python binding gives serves M Hq <= 496.
-//   More rows from M Hq keys of 560 K: 16 / 2 heads, 48 tokens on 256 cached 9.5 -> 11.5, on 512 11.0 -> 11.9, on 1500 16.4
-//   -> 14.8; 64 tokens 5.5 -> 7.7, on 256 cached 10.3 -> 11.8, on 512 12.2 level, on 1000 15.8 -> 14.6; 128 tokens, which
-//   stay below it, 10.6 -> 8.6, on 128 13.0 -> 10.7, on 512 18.1 -> 15.1.
-// attn_bound_from: the keys from which a call's bound on them lets attend_prompt serve it (0: never). attn_keys_from: those
-// from which, in attention_select, it then does (one token 50 K Hq keys, few rows 76 K M Hq keys, up to 383 rows 2048 keys,
-// beyond 192: where the two bodies crossed in sweeps of 200 .. 16000 keys on 4096- to 16384-row caches).
+//   More rows, us: 65 to 128 keys, which attention_mfma splits and attend_prompt need not (16 / 2 heads, 64 tokens on 64
+//   cached 9.0 -> 8.5, 128 tokens 10.6 -> 8.5; up to 64 keys neither does, 64 tokens 5.5 -> 7.7). Up to 383, where
+//   attend_prompt's one walk of the keys grows with them and the other's with the rows, from M Hq of 4 keys + 256 (16 / 2
+//   heads, 64 tokens on 128 cached 9.2 -> 9.4, 80 on 128 10.4 -> 10.1, 64 on 256 10.3 -> 11.0, 128 on 128 12.9 -> 10.1; 12 /
+//   2, 86 on 128 9.9 -> 10.1, 107 on 128 10.5 -> 10.1; 28 / 4, 64 on 128 11.5 -> 9.5). Beyond, from M Hq keys of 700 K (48
+//   tokens on 512 cached 11.0 -> 11.9, on 1500 16.4 -> 14.8; 64 on 512 12.2 level, on 1000 15.8 -> 14.6; 4 / 4 heads, 384
+//   on 64 12.6 -> 13.1, on 128 13.7 -> 13.1).
+// attn_bound_from: the keys from which a call's bound on them lets attend_prompt serve few rows (0: never), attn_prompt_bound
+// whether it lets it serve more. attn_keys_from: the keys from which, in attention_select, it then does (one token 50 K Hq
+// keys, few rows 76 K M Hq keys, up to 383 rows 2048 keys, beyond 192: where the two bodies crossed in sweeps of 200 ..
+// 16000 keys on 4096- to 16384-row caches).
+bool attn_prompt_bound(long work, int max_keys) {
+  if (max_keys >= kAttnPromptSplitKeys) return work * max_keys >= kAttnPromptWork;
+  return max_keys > 64 && (max_keys <= 128 || work >= 4L * max_keys + 256);
+}
 int attn_bound_from(int M, int Hq, int Hkv, size_t ws_bytes) {
   const int G = Hq / Hkv;
   const long rows = (long)M * G, work = (long)M * Hq;
-  if (rows >= kAttnPromptMinRows) return (int)std::max<long>(1, (kAttnPromptWork + work - 1) / work);
   if (G == 1 && rows < 16) return 0;
   if (rows < kAttnMfmaMinRows && (long)M * Hkv >= 64) return 0;
   if (ws_bytes < kAttnCounterBytes + (size_t)16 * M * Hq * kAttnRec * sizeof(float)) return 0;
@@ -1308,8 +1326,19 @@ hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int6
                             int Hkv, int L, int max_keys, float scale, void* ws, size_t ws_bytes, hipStream_t st) {
   const long rows = (long)M * (Hq / Hkv);
   if (!ws) ws_bytes = 0;
+  const int from = attn_keys_from(M, Hq, Hkv);
+  if (rows >= kAttnPromptMinRows) {
+    if (!attn_prompt_bound((long)M * Hq, max_keys))
+      return launch_attention_mfma(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+    // M tokens attend M keys at least, unless they share positions; a bound of more may lie far above them
+    const bool sure = M >= from, wide = (rows + 63) / 64 * Hkv < kAttnPromptWide;
+    if (max_keys < kAttnPromptLongKeys || (sure && !wide && prompt_parts<2, 2>(M, Hq, Hkv, max_keys, ws, ws_bytes, 512) == 1))
+      return launch_attention_prompt(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
+    if (wide)
+      return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, sure ? 1 : from);
+    return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, sure ? 1 : from);
+  }
   const int bound_from = attn_bound_from(M, Hq, Hkv, ws_bytes);
-  int from = attn_keys_from(M, Hq, Hkv);
   if (bound_from > 0 && max_keys >= bound_from) {
     if (rows < kAttnMfmaMinRows)
       return launch_attention_select<2, 2, true>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
@@ -1317,14 +1346,7 @@ hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int6
     // 24000: 24 against 27)
     if (rows <= 128)
       return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
-    if (rows < kAttnPromptMinRows)
-      return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
-    if (max_keys < kAttnPromptLongKeys)
-      return launch_attention_prompt(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);
-    if (M >= from) from = 1;                                  // (M tokens attend M keys at least, unless they share positions)
-    if ((rows + 63) / 64 * Hkv < kAttnPromptWide)
-      return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, from);
-    return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 512, from);
+    return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
   }
   if (rows >= kAttnMfmaMinRows)
     return launch_attention_mfma(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st);

@@ -283,11 +283,12 @@ constexpr size_t kAttnCounterBytes = 4096;
 // splits keys while its waves number fewer than kAttnMfmaTargetWaves
 constexpr int kAttnMfmaMinRows = 32;
 constexpr int kAttnMfmaTargetWaves = 512;
-// the prompt attention (decode_ops.hip, attn_bound_from): steps of kAttnPromptMinRows or more query rows per KV head from
-// kAttnPromptWork (token, head, key)s, of fewer from kAttnLongKeys keys and kAttnLongWork(One); with 64 rows a workgroup, or
-// 32 where those leave CUs idle (fewer than kAttnPromptWide workgroups) and a bound of kAttnPromptLongKeys keys or more
+// the prompt attention (decode_ops.hip, attn_bound_from and attn_prompt_bound): steps of kAttnPromptMinRows or more query rows
+// per KV head, where the keys are split from kAttnPromptWork (token, head, key)s, and of fewer rows from kAttnLongKeys keys
+// and kAttnLongWork(One); with 64 rows a workgroup, or 32 where those leave CUs idle (fewer than kAttnPromptWide workgroups)
+// and a bound of kAttnPromptLongKeys keys or more
 constexpr int kAttnPromptMinRows = 384;
-constexpr long kAttnPromptWork = 560000;
+constexpr long kAttnPromptWork = 700000;
 constexpr int kAttnPromptWide = 160;
 constexpr int kAttnPromptLongKeys = 1024;
 constexpr int kAttnLongKeys = 2048;
