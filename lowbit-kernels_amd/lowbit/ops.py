@@ -196,12 +196,13 @@ def auto_version(m, wq):
     return None
 
 
-def prefill(x, wq, own_workspace=False):
+def prefill(x, wq):
     """x [M, K] times an mma-layout weight with the int4-direct prefill GEMM (any M; fp32 accumulation of exactly the
-    dequantized fp16 weights, as dequantize + BLAS computes). own_workspace: see w4_gemm_prefill."""
+    dequantized fp16 weights, as dequantize + BLAS computes)."""
     if wq.packed_mma is None:
         raise ValueError("the prefill GEMM reads packed_mma, which this W4Weight does not keep")
-    return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, own_workspace=own_workspace)
+    return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group,
+                                 own_workspace=_own_workspace(x.shape[0], wq))
 
 
 def _prefill_without_blas(m, wq):
@@ -209,6 +210,12 @@ def _prefill_without_blas(m, wq):
     calls that torch differentiates or transforms (_plain)."""
     return (wq.k >= AUTO_PREFILL_MIN_K or m <= AUTO_PREFILL_ROWS
             or (m <= AUTO_PREFILL_NARROW_ROWS and wq.n <= AUTO_PREFILL_NARROW and wq.k <= AUTO_PREFILL_NARROW))
+
+
+def _own_workspace(m, wq):
+    """Calls that BLAS would serve, were they not plain, share no scratch when they are captured on one stream, as BLAS
+    calls do not."""
+    return not _prefill_without_blas(m, wq)
 
 
 def prefill_path(m, wq):
@@ -281,12 +288,10 @@ def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     if v is not None:
         y = gemv(x, wq, v)
     elif version == 0 and prefill_path(m, wq) and (_prefill_without_blas(m, wq) or _plain(x, given)):
-        # beyond _prefill_without_blas, calls captured on one stream share no scratch, as BLAS calls do not
-        own = not _prefill_without_blas(m, wq)
         if bias is not None:
             return ext().w4_gemm_prefill(x.contiguous(), wq.packed_mma, wq.scales, wq.group, _native.EPI_BIAS, bias,
-                                         own_workspace=own)
-        y = prefill(x, wq, own)
+                                         own_workspace=_own_workspace(m, wq))
+        y = prefill(x, wq)
     else:
         y = torch.nn.functional.linear(x, dequant(wq, "mma" if wq.packed_mma is not None else "canonical"))
     return y.add_(bias) if bias is not None else y

@@ -23,7 +23,7 @@ def layer(monkeypatch):
             taken.append(name)
             return result(*args, **kwargs)
         return call
-    monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq, own: x.detach() @ w.t()))
+    monkeypatch.setattr(ops, "prefill", fake("prefill", lambda x, wq: x.detach() @ w.t()))
     monkeypatch.setattr(ops, "dequant", fake("dequant", lambda *a: w))
     monkeypatch.setattr(ops, "ext", lambda: SimpleNamespace(w4_gemm_prefill=fake(
         "prefill+bias", lambda x, p, s, g, epilogue, bias, **own: (x.detach() @ w.t()).add_(bias.detach()))))
