@@ -247,11 +247,15 @@ int lowbit_w4_qkv_rope_rows(const void* x, const void* w, const void* s, int64_t
                             void* workspace, size_t workspace_bytes, void* stream);
 
 /* Causal GQA attention: out[M][Hq * 128] for queries q [M][Hq][128] at positions[m] over cache rows 0..positions[m]
- * (at most L); scores scaled by `scale`, softmax and P.V in fp32. Cache rows past the largest position of the call
+ * (at most L); scores scaled by `scale`, softmax and the sums of P.V in fp32. The kernels on matrix cores (32 or more
+ * query rows per KV head, and fewer on long contexts) split each softmax weight in P.V into an fp16 head and remainder,
+ * good to ~2^-22 of the weight and to no less than 2^-25 of the largest (2^-32 in the long-context and prompt kernel, 2^-39
+ * there below 32 rows). Cache rows past the largest position of the call
  * are never read into a result (they may hold anything, NaN included); rows up to it must be finite, since a
- * multi-token step reads whole blocks of keys up to the largest position of the rows it groups. max_keys: an upper bound on positions[m] + 1 over
- * the calls that will run (sizes the launch; a captured graph keeps it; keys past it are still attended, by the last
- * key partition). Hq / Hkv in {1, 2, 4, 6, 7, 8}. workspace (optional, 16-byte aligned, at least 4096 bytes, no
+ * multi-token step reads whole blocks of keys up to the largest position of the rows it groups. max_keys: an upper bound
+ * on positions[m] + 1 over the calls that will run (sizes the launch; a captured graph keeps it; keys past it are still
+ * attended). Under a bound of a long context each call picks its kernel and key partitions on the GPU by positions[M - 1];
+ * a bound near the real count saves a launch on short contexts. Hq / Hkv in {1, 2, 4, 6, 7, 8}. workspace (optional, 16-byte aligned, at least 4096 bytes, no
  * initial contents needed; its first 4096 bytes are not used -- version 0.2 kept arrival counters there and needed
  * them zero): when there are too few (token, head group) blocks to fill the GPU and max_keys >= 512, the keys are
  * split into partitions whose fp32 partial softmax sums (blocks x partitions x (2 + 128) x 4 bytes after the first
@@ -269,11 +273,12 @@ int lowbit_attention(const void* q, const void* k_cache, const void* v_cache, co
  * attention keeps at most 8 key partitions and leaves their partial softmax sums in the workspace; the projection's
  * prologue merges them into its x in partition order, the attention's own merge, so y has the bits of lowbit_attention
  * (with a workspace that holds at most the same partitions) followed by lowbit_w4_linear_fused / lowbit_f16_linear_fused
- * at M = 1 -- one launch fewer, and the attention output never written. On a long cache (Hq * max_keys >= 128000 and a
- * workspace of 16 partitions or more) the attention splits the keys further and merges them itself, as lowbit_attention
- * does there: three launches, the bits of lowbit_attention with a workspace smaller by Hq * 256 bytes. Hq <= 32, Hq / Hkv in {1, 2, 4, 6, 7, 8};
- * workspace required: 16-byte aligned, at least 4096 + Hq * 132 * 4 bytes, no initial contents (the partials, P x Hq
- * x 132 x 4 bytes, follow its first 4096). No counterpart in the reference (its decoder runs torch attention, then
+ * at M = 1 -- one launch fewer, and the attention output never written. Under the bound of a long cache (max_keys >= 2048, Hq *
+ * max_keys >= 128000, two or more query heads per KV head, and a workspace of 16 partitions or more) the attention merges
+ * its partitions itself, as lowbit_attention does there: three launches, the bits of lowbit_attention with a workspace
+ * smaller by Hq * 256 bytes. Hq <= 32, Hq / Hkv in {1, 2, 4, 6, 7, 8}; workspace required: 16-byte aligned, at least
+ * 4096 + Hq * 132 * 4 bytes, no initial contents (the partials, P x Hq x 132 x 4 bytes, follow its first 4096). No
+ * counterpart in the reference (its decoder runs torch attention, then
  * W4Linear); it serves the fused decoder's one-token step. */
 int lowbit_w4_attention_linear(const void* q, const void* k_cache, const void* v_cache, const int64_t* positions,
                                int64_t Hq, int64_t Hkv, int64_t L, int64_t max_keys, float scale, const void* w,

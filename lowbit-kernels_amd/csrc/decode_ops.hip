@@ -536,8 +536,8 @@ __global__ __launch_bounds__(64) void attention_mfma(const f16* __restrict__ q, 
 // workgroup at KG = 2). Against 64 rows (RG = KG = 2), 128 rows (RG = 4, KG = 1) lengthen the serial walk of the last
 // rows: 3000 tokens 97 us against 81 (before K's second block ahead and the transposing reads), 700 tokens 27 against
 // 21; 32 rows (KG = 4) double the L2 reads (126 us) and win only where 64 rows leave CUs idle.
-// MI355X, 16 query / 2 KV heads, us (attention_mfma -> this): 3000 tokens 285 -> 76, 700 tokens 32.5 -> 17.2, 300 tokens
-// 16.4 -> 11.4, 128 tokens 11.1 -> 8.9; 512 tokens on 4096 cached 204 -> 53, 128 on 8000 125 -> 39 (KG = 4; 70 and 49
+// MI355X, 16 query / 2 KV heads, graph-timed, us (attention_mfma -> this): 3000 tokens 283 -> 73, 700 tokens 34.5 -> 17.1,
+// 300 tokens 16.1 -> 11.4, 128 tokens 10.9 -> 8.7; 512 tokens on 4096 cached 203 -> 51, 128 on 8000 125 -> 39 (KG = 4; 70 and 49
 // with KG = 2); 28 / 4 heads, 2048 tokens 230 -> 63.
 constexpr float kAttnLagFew = 1.f, kAttnLag = 8.f;
 

@@ -21,9 +21,10 @@
 // whole, fragment reads waited for as they were issued, x through registers, a barrier that drained every load) left the
 // matrix cores 31% busy at 2048 x 3584 x 18944; this one keeps them 45-50% busy there, at the clock that the power limit
 // leaves (1.8-2.0 GHz; MFMAs with the decode's vector instructions between them and nothing else reach 1.6 PFLOP/s).
-// MI355X, graph-timed, cold weights, rows x K x N, us (before -> now, dequantize + hipBLASLt): 128 x 3584 x 18944 37.9 ->
-// 28.7 (63.5); 333 x 2048 x 11008 32.6 -> 30.3 (41.6); 333 x 11008 x 2048 46.8 -> 30.7 (52.4); 512 x 18944 x 3584 104 ->
-// 84 (203); 700 x 2048 x 22016 81 -> 73 (102); 1000 x 3584 x 18944 182 -> 149 (164); 2048 x 3584 x 18944 354 -> 282 (341).
+// MI355X, graph-timed, cold weights, one run, rows x K x N, us (before -> now, dequantize + hipBLASLt): 128 x 3584 x 18944
+// 42.8 -> 36.8 (67.3); 333 x 2048 x 11008 34.4 -> 32.2 (43.5); 333 x 11008 x 2048 49.1 -> 37.0 (55.1); 512 x 18944 x 3584
+// 111 -> 87 (204); 700 x 2048 x 22016 90 -> 75 (106); 1000 x 3584 x 18944 184 -> 140 (161); 2048 x 3584 x 18944 334 -> 258
+// (341).
 // Not kept: the same loop on 32x32x16 MFMAs (271-294 at 2048 x 3584 x 18944, more power per product), 8 tiles x 4
 // per wave (registers spill; the compiler moves accumulators between register files at 16), 8-wave workgroups.
 //
@@ -366,10 +367,11 @@ hipError_t launch_prefill(const GemvArgs& a, const PrefillPlan& p, uint32_t* ctr
 // The tile shapes built, and what a launch of each costs (us): `groups` workgroups share a CU (registers, LDS); `base` for
 // a launch; a workgroup takes `alone` per 128-k chunk, or a CU's resident ones `each` per chunk and workgroup when that is
 // more; a K split costs `split` and `per_mb` per MB of partials. Fitted to an MI355X sweep (graph-timed, cold weights, 65
-// to 2048 rows of 12 Qwen2.5-0.5B .. 7B projections, 1 to 8 splits; the fit's error is 10-15%); the cheapest plan by it
-// is 2.5% slower than the sweep's best on average and 26% at worst. `alone` of the 64-row shapes was raised from the fit's
-// 0.74 and 0.66 afterwards: a workgroup that has its CU to itself and walks all of K waits for its weights (0.86 .. 0.9 a
-// chunk), so two splits beat it (2048 x 2048 at 512 rows 17.0 -> 14.2, 2048 x 2560 at 300 17.0 -> 14.2, 3584 x 4608 at 333
+// to 2048 rows of 12 Qwen2.5-0.5B .. 7B projections, 1 to 8 splits; the fit's error is 10-15%); the cheapest plan by
+// the fitted constants was 2.5% slower than the sweep's best on average and 26% at worst. `alone` of the 64-row shapes was
+// raised from the fit's 0.74 and 0.66 afterwards, by the points named here and without taking those two figures again: a
+// workgroup that has its CU to itself and walks all of K waits for its weights (0.86 .. 0.9 a chunk), so two splits beat it
+// (2048 x 2048 at 512 rows 17.0 -> 14.2, 2048 x 2560 at 300 17.0 -> 14.2, 3584 x 4608 at 333
 // 28.1 -> 25.1, 3584 x 3584 at 400 27.8 -> 24.9, 1536 x 2048 at 512 13.0 -> 12.1).
 struct PrefillShape {
   int MT, PT, groups;

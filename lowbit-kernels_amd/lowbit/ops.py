@@ -166,13 +166,13 @@ AUTO_GEMV_NARROW_ROWS, AUTO_GEMV_NARROW_N, AUTO_GEMV_MAX_K = 3, 8192, 16384
 # AUTO_PREFILL_NARROW), and up to as many where the BLAS GEMM's 256 x 256 tiles, more than one round of the 256 CUs, would
 # fill its rounds to less than AUTO_PREFILL_FILL; everything else dequantizes (4.4-4.8 TB/s) and calls BLAS. From an
 # MI355X sweep of 65 .. 2048 rows on 12 Qwen2.5-0.5B .. 7B projections (int4 vs dequantize + hipBLASLt, us): every layer
-# up to 1000 rows (2048 x 22016 20 vs 42 at 128, 56 vs 73 at 512, 96 vs 114 at 1000; 3584 x 18944 29 vs 63, 76 vs 99, 149
-# vs 164; 11008 x 2048 19 vs 35, 37 vs 54, 62 vs 73; layers of 4096 < N <= 8192, of which the sweep has one, keep the
-# older 512); the small layers at 2048 (2048 x 2048 25 vs 31, 3584 x 3584 57 vs 59) and the long-K 7B down at every M (279
-# vs 396 at 2048). At 1400 and 2048 rows the fill decides: 0.67 .. 0.77 of the rounds 2048 x 22016 at 1400 133 vs 145,
-# 3584 x 18944 at 2048 282 vs 341, 1536 x 17920 at 2048 123 vs 134; 0.86 .. 0.9 3584 x 18944 at 1400 196 vs 187, 2048 x
-# 22016 at 2048 200 vs 188; 1.0 3584 x 16384 at 2048 245 vs 205; under one round (narrow layers, where BLAS takes smaller
-# tiles) 11008 x 2048 at 2048 110 vs 104, 8960 x 1536 73 vs 72.
+# up to 1000 rows (2048 x 22016 23 vs 46 at 128, 60 vs 75 at 512, 96 vs 114 at 1000; 3584 x 18944 35 vs 64, 78 vs 101, 140
+# vs 161; 11008 x 2048 20 vs 38, 39 vs 58, 62 vs 73; layers of 4096 < N <= 8192, of which the sweep has one, keep the
+# older 512); the small layers at 2048 (2048 x 2048 25 vs 32, 3584 x 3584 57 vs 59) and the long-K 7B down at every M (284
+# vs 392 at 2048). At 1400 and 2048 rows the fill decides: 0.67 .. 0.77 of the rounds 2048 x 22016 at 1400 133 vs 145,
+# 3584 x 18944 at 2048 267 vs 341, 1536 x 17920 at 2048 123 vs 134; 0.86 .. 0.9 3584 x 18944 at 1400 196 vs 187, 2048 x
+# 22016 at 2048 189 vs 191 (200 vs 188 on another box); 1.0 3584 x 16384 at 2048 245 vs 205; under one round (narrow layers, where BLAS takes smaller
+# tiles) 11008 x 2048 at 2048 115 vs 106, 8960 x 1536 73 vs 72. No fill between 0.77 and 0.86 was measured; 0.8 is halfway.
 AUTO_PREFILL_MIN_K, AUTO_PREFILL_ROWS = 16384, 512
 AUTO_PREFILL_WIDE_N, AUTO_PREFILL_WIDE_ROWS = 8192, 1024
 AUTO_PREFILL_NARROW, AUTO_PREFILL_NARROW_ROWS = 4096, 2048
@@ -261,7 +261,11 @@ def _plain(x, bias=None):
 def linear(x, wq, max_gemv_rows=8, version=0, bias=None):
     """Decode (few rows): an INT4 kernel (v6 GEMV for one row, v5 MFMA beyond). Prefill (many rows): dequantize, then
     the fp16 BLAS GEMM (hipBLASLt under PyTorch-ROCm), or the int4 prefill GEMM where prefill_path says (K >=
-    AUTO_PREFILL_MIN_K at any M, every layer up to AUTO_PREFILL_ROWS rows, some up to AUTO_PREFILL_NARROW_ROWS). version 0 = auto; a fixed version runs up to min(max_gemv_rows, its row
+    AUTO_PREFILL_MIN_K at any M, every layer up to AUTO_PREFILL_ROWS rows, some up to AUTO_PREFILL_NARROW_ROWS). Of those,
+    the calls that only BLAS served before keep it where torch differentiates, transforms or traces them, under a mode or
+    autocast, and where x does not start on a 16-byte boundary (_plain); captured, they keep their scratch in their graph,
+    while the others use their stream's, so graphs that hold such calls and were captured on one stream must not run at
+    the same time. version 0 = auto; a fixed version runs up to min(max_gemv_rows, its row
     limit) rows (v5: 64), and dequantize + BLAS above.
     bias ([N], optional; not in the reference's signature; used in fp16 on x's device on every route): y =
     fp16(x W^T) + bias in fp16, the rounding of the reference's linear() followed by `+ bias`; the v5, one-row v6 and prefill kernels add it in their store (no extra
