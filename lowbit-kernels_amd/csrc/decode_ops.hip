@@ -1342,8 +1342,8 @@ hipError_t attention_launch(const f16* q, const f16* k, const f16* v, const int6
   if (bound_from > 0 && max_keys >= bound_from) {
     if (rows < kAttnMfmaMinRows)
       return launch_attention_select<2, 2, true>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
-    // 64 rows a workgroup up to 128 rows, 32 beyond (28 / 4 heads, 32 tokens on 24000: 43 us against 53; 16 / 2, 16 on
-    // 24000: 24 against 27)
+    // 64 rows a workgroup up to 128 rows, 32 beyond (28 / 4 heads, 32 tokens on 24000, in a workspace that holds their
+    // partitions: 43 us against 53; 16 / 2, 16 on 24000: 24 against 27)
     if (rows <= 128)
       return launch_attention_select<2, 2, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
     return launch_attention_select<1, 4, false>(q, k, v, pos, out, M, Hq, Hkv, L, max_keys, scale, ws, ws_bytes, st, 256, from);
