@@ -102,7 +102,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const void* __restrict__ 
 // scale, whose reciprocal says nothing, and a group whose largest quotient overflows (a clip factor near 0 on weights near
 // fp32's largest; q0 would be infinite and r not a number) take the division itself.
 // Bound: vector instructions (8 per value and candidate; the division took ~10 by itself). 11008 x 2048 fp16, 11
-// candidates, MI355X: quantize_kernel 208 us, 72 here.
+// candidates, MI355X: quantize_kernel 207 us, 63 here.
 template <int kDtype>
 __device__ __forceinline__ void load8(const void* w, size_t i, float (&v)[8]) {
   if constexpr (kDtype == 0) {
